@@ -11,59 +11,15 @@
 // than one block loop over blocks.  At GPT-2's per-layer sizes (0.6 to 4.7 MB of weights) a
 // call is bound by launch and memory latency, and one row per wave gives the most waves; a
 // tall matrix (50304 x 768) streams, and 2-4 rows per wave keep 3-6 KB per wave in flight.
-// MFMA is not used (B is a handful of decode tokens, 1-2 flops per byte).
-#include <hip/hip_runtime.h>
-#include <math.h>
-#include <stdint.h>
-
-#include "kvattn.h"
-#include "lanes.hpp"
+// Batches of tokens take the matrix cores (gemm.hip) where those are faster (gemm_takes); the time
+// here grows with the number of vectors.
+#include "fc.hpp"
 
 namespace {
 
 constexpr int kGemvWaves = 4;          // waves per workgroup
 constexpr int kGemvMaxChunks = 16;     // 16-byte weight chunks per lane and row in one block
 constexpr int kGemvMaxRowChunks = 16;  // kR * kC: weight registers of a wave (64 VGPRs)
-
-template <int WT> struct WFmt;
-template <> struct WFmt<KVATTN_KV_F32> {   // x, bias, out: float
-    static constexpr int kWBytes = 4, kElems = 4, kXBytes = 16;
-    static constexpr bool kActF32 = true, k8bit = false;
-};
-template <> struct WFmt<KVATTN_KV_BF16> {  // x, bias, out: bf16
-    static constexpr int kWBytes = 2, kElems = 8, kXBytes = 16;
-    static constexpr bool kActF32 = false, k8bit = false;
-};
-template <> struct WFmt<KVATTN_KV_INT8> {  // x, bias, out: bf16
-    static constexpr int kWBytes = 1, kElems = 16, kXBytes = 32;
-    static constexpr bool kActF32 = false, k8bit = true;
-};
-template <> struct WFmt<KVATTN_KV_FP8_E4M3> {
-    static constexpr int kWBytes = 1, kElems = 16, kXBytes = 32;
-    static constexpr bool kActF32 = false, k8bit = true;
-};
-
-struct GemvArgs {
-    void* out;
-    void* pre_gelu;
-    const uint8_t* W;
-    const float* w_scale;
-    const uint8_t* x;
-    const void* bias;
-    int B, M, K, gelu;
-    // QKV projection with the KV append in its epilogue (kv != nullptr): out is qkv
-    // [B][3][NH][64], and its K and V rows also go to column cur_len of the cache
-    // [2][B][NH][maxT][64], in the activation type or (kv_dtype 8-bit) as codes with a row
-    // scale in kv_scale [2][B][NH][maxT].  8-bit rows pass through `words` (tagged u64
-    // [B][2][NH][64]), their wait bounded by `polls`.
-    uint8_t* kv;
-    const int* cur_len;
-    int lens_per_seq, NH, maxT;
-    int kv_dtype;
-    float* kv_scale;
-    unsigned long long* words;
-    int polls;
-};
 
 // The x values one 16-byte weight chunk multiplies: 16 bytes (4 floats or 8 bf16), or 32
 // bytes (16 bf16) for 8-bit weights.
@@ -118,49 +74,11 @@ __device__ __forceinline__ float chunk_dot(const uint4& w, const XRaw<WT>& xr) {
     return s;
 }
 
-template <int WT>
-__device__ __forceinline__ float load_act(const void* p, size_t i) {
-    if constexpr (WFmt<WT>::kActF32) return reinterpret_cast<const float*>(p)[i];
-    else return bf16_to_f32(reinterpret_cast<const uint16_t*>(p)[i]);
-}
-
-template <int WT>
-__device__ __forceinline__ void store_act(void* p, size_t i, float v) {
-    if constexpr (WFmt<WT>::kActF32) reinterpret_cast<float*>(p)[i] = v;
-    else reinterpret_cast<uint16_t*>(p)[i] = f32_to_bf16(v);
-}
-
-// out / pre_gelu element: float or bf16 (the output type may differ from the activations,
-// as in the reference's float logits over bf16 activations).
-template <bool kOutF32>
-__device__ __forceinline__ void store_res(void* p, size_t i, float v) {
-    if constexpr (kOutF32) reinterpret_cast<float*>(p)[i] = v;
-    else reinterpret_cast<uint16_t*>(p)[i] = f32_to_bf16(v);
-}
-
-// GPT-2's GELU, tanh form: 0.5 v (1 + tanh(sqrt(2/pi) (v + 0.044715 v^3))).
-__device__ __forceinline__ float gelu_tanh(float v) {
-    const float cube = 0.044715f * v * v * v;
-    return 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + cube)));
-}
-
-constexpr int kHd = 64;   // head size of the QKV epilogue
 constexpr int kHeadRowGroups = kHd / kGemvWaves;   // workgroups of one head row (64 channels, one row per wave)
-// The epilogue of a launch (a template parameter, so that the plain GEMV carries none of it).
-enum GemvEpilogue { kEpiNone = 0, kEpiAppend = 1, kEpiAppend8 = 2 };
-// Bits of the preloaded M argument above the row count (M < 2^29): GELU, and the XCD-local
-// layout of kEpiAppend8.
-constexpr int kGeluFlag = 1 << 29, kXcdLocalFlag = 1 << 30, kRowMask = (1 << 29) - 1;
 
-// Cache row (in units of kHd elements) of part 1 (K) or 2 (V), head h, sequence b at the
-// position being appended: column cur_len, clamped to [0, maxT - 1] as the append does.
-// len0: cur_len[0], loaded ahead with the weights.
+// cache_row_at with the length read here; len0: cur_len[0], loaded ahead with the weights.
 __device__ __forceinline__ size_t cache_row(const GemvArgs& a, int b, int part, int h, int len0) {
-    int cl = a.lens_per_seq && b > 0 ? a.cur_len[b] : len0;
-    cl = cl < 0 ? 0 : (cl > a.maxT - 1 ? a.maxT - 1 : cl);
-    size_t row = ((size_t)b * a.NH + h) * a.maxT + cl;
-    if (part == 2) row += (size_t)a.B * a.NH * a.maxT;
-    return row;
+    return cache_row_at(a, b, part, h, a.lens_per_seq && b > 0 ? a.cur_len[b] : len0);
 }
 
 // The weights, x, scales, bias, shape and output also come as leading scalar parameters
@@ -412,11 +330,6 @@ const void* gemv_ptr_out(int chunks_per_lane, int rows, bool out_f32, int epi) {
 
 }  // namespace
 
-namespace kvattn_internal {
-void set_last_hip_error(int e);   // kvattn.hip: read back by kvattn_last_hip_error
-int merge_poll_limit();           // kvattn.hip: kvattn_set_merge_poll_limit's bound
-}
-
 namespace {
 
 // Checks shared by the entry points, then the launch.  out_f32: out and pre_gelu as float,
@@ -438,6 +351,10 @@ int launch_gemv(GemvArgs a, int w_dtype, bool out_f32, void* stream) {
         ((uintptr_t)a.w_scale & 3u) ||
         (a.kv && a.kv_dtype != KVATTN_KV_INT8 && a.kv_dtype != KVATTN_KV_FP8_E4M3 && ((uintptr_t)a.kv % act)))
         return KVATTN_ERR_MISALIGNED;
+    const bool kv8 = a.kv && (a.kv_dtype == KVATTN_KV_INT8 || a.kv_dtype == KVATTN_KV_FP8_E4M3);
+    const int epi = !a.kv ? kEpiNone : (kv8 ? kEpiAppend8 : kEpiAppend);
+    if (kvattn_internal::gemm_takes(w_dtype, B, M, K))
+        return kvattn_internal::launch_gemm(a, w_dtype, out_f32, epi, stream);
     const int nch = K * wbytes / 16;
     const int per_lane = (nch + kWave - 1) / kWave;
     // Measured at 50304 x 768 (per call, graph of calls over weights beyond the Infinity
@@ -446,8 +363,6 @@ int launch_gemv(GemvArgs a, int w_dtype, bool out_f32, void* stream) {
     // 8 rows 9.8 / 15.5 / 24.9; one row 16.8 / 19.0 / 26.6.  Workgroups of 8 or 16 waves
     // instead of 4: +0.5 to +2.6 us.  The QKV epilogue takes one row per wave.
     const int rows = a.kv || M < kGemvTallRows ? 1 : (w8 ? 4 : 2);
-    const bool kv8 = a.kv && (a.kv_dtype == KVATTN_KV_INT8 || a.kv_dtype == KVATTN_KV_FP8_E4M3);
-    const int epi = !a.kv ? kEpiNone : (kv8 ? kEpiAppend8 : kEpiAppend);
     const void* fn = nullptr;
     switch (w_dtype) {
         case KVATTN_KV_F32: fn = gemv_ptr_out<KVATTN_KV_F32>(per_lane, rows, out_f32, epi); break;

@@ -373,9 +373,11 @@ int kvattn_paged_decode(void* out, const void* qkv, void* pages, float* page_sca
  * projection), each wave takes 4 rows so that more weight bytes are in flight.
  * Replaces launch_GEMV6_fused (Inference_gpt2/GEMV.cuh:132-206) and launch_GEMV6_w8x2
  * (Inference_gpt2/GEMV_w8.cuh:64-184), which matmul_forward[_w8] calls for one decode token
- * (inference_gpt2_opt.cu:106-132); the attention output projection is at :349-355.  B > 1
- * reads the weights once for all B vectors when a row fits in one block (the reference
- * takes cuBLASLt there). */
+ * (inference_gpt2_opt.cu:106-132); the attention output projection is at :349-355.  Batches
+ * (from 3 vectors on, FP32 weights from 4 or 8, up to 8191 rows) go through the matrix cores with
+ * FP32 sums, where the reference takes cuBLASLt; other B > 1 read the weights once for all B
+ * vectors when a row fits in one block.  A vector's result may differ in its last bits with
+ * the size of the batch (another order of the same sums). */
 int kvattn_gemv(void* out, void* pre_gelu, const void* W, const float* w_scale, const void* x,
                 const void* bias, int B, int M, int K, int w_dtype, int gelu, void* stream);
 
@@ -395,7 +397,8 @@ int kvattn_gemv_ex(void* out, void* pre_gelu, const void* W, const float* w_scal
  *     otherwise); kv_scale and the workspace are not used.
  *   kv_dtype INT8 / FP8_E4M3 (bf16 activations): codes and one row scale per (b, K|V, h) in
  *     kv_scale [2][B][NH][maxT], from the bf16 values in qkv with the append's quantiser.
- *     The 64 channels of a row come from 16 workgroups, so they meet in the workspace:
+ *     On the vector units the 64 channels of a row come from 16 workgroups, so they meet
+ *     in the workspace (a batch on the matrix cores does not use it, but it is checked alike):
  *     kvattn_gemv_qkv_append_workspace_bytes(B, NH) bytes, 256-byte aligned, zeroed once
  *     (kvattn_workspace_init); each word there carries the call that wrote it, so the
  *     workspace needs no clearing between calls.  Calls sharing a workspace must be ordered

@@ -1,0 +1,122 @@
+"""GPU tests of the matrix-core path of kvattn_gemv (batches of tokens) and of
+kvattn_gemv_qkv_append on it.
+
+Bound: FP32 sums of exact products in any order differ from the exact sum by at most
+(K + 8) 2^-24 sum |w x| (the row scale, the bias and the output's rounding included in the 8),
+which _bound computes for every output; float outputs are asked for, so nothing else rounds.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from tests.test_gpu_gemv import _kv, _make, _run
+
+pytestmark = pytest.mark.gpu
+
+
+def _bound(h, B, M, K):
+    W, x = np.abs(h["W"]).reshape(M, K).astype(np.float64), np.abs(h["x"]).reshape(B, K).astype(np.float64)
+    s = np.ones(M) if h["scale"] is None else np.abs(h["scale"]).astype(np.float64)
+    b = np.zeros(M) if h["bias"] is None else np.abs(h["bias"]).astype(np.float64)
+    return (K + 8) * 2.0 ** -24 * ((x @ W.T) * s + b)
+
+
+def _exact(h, B, M, K):
+    y = h["x"].reshape(B, K).astype(np.float64) @ h["W"].reshape(M, K).astype(np.float64).T
+    y = y if h["scale"] is None else y * h["scale"].astype(np.float64)
+    return y if h["bias"] is None else y + h["bias"].astype(np.float64)
+
+
+def _guarded(t):
+    """The same values, followed in memory by NaNs (NaN codes)."""
+    import torch
+    flat = t.reshape(-1)
+    fill = torch.full((4096,), 0x7F if t.dtype == torch.uint8 else float("nan"), dtype=t.dtype)
+    return torch.cat([flat, fill])
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "int8", "fp8"])
+@pytest.mark.parametrize("B,M,K", [(4, 1, 16), (8, 15, 48), (15, 16, 64), (16, 17, 80), (17, 63, 784), (33, 130, 768),
+                                   (64, 40, 1040), (9, 8191, 32), (40, 33, 5136)])
+def test_batch_against_float64(dev, dtype, B, M, K):
+    """Tiles of 16 rows x 16 tokens that are full, one short and one over; rows of one chunk, of a
+    partial last step, of fewer steps than waves and of several blocks of loads; NaNs right
+    behind the weights and the tokens."""
+    d, h = _make(dtype, B, M, K, seed=B * 1000 + M + K)
+    d = dict(d, W=_guarded(d["W"]), x=_guarded(d["x"]))
+    got, _ = _run(d, dtype, B, M, K, False, False, out_dtype="f32")
+    err = np.abs(got.reshape(B, M).astype(np.float64) - _exact(h, B, M, K))
+    assert np.all(err <= _bound(h, B, M, K)), float((err / _bound(h, B, M, K)).max())
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "int8", "fp8"])
+def test_batch_gelu_and_pre_gelu(dev, dtype):
+    B, M, K = 19, 200, 304
+    d, h = _make(dtype, B, M, K, seed=77)
+    got, pre = _run(d, dtype, B, M, K, True, True)
+    ref, rpre = oracle.gemv(h["W"], h["x"], B, M, K, w_scale=h["scale"], bias=h["bias"], gelu=True, want_pre=True)
+    tol = 1e-5 if dtype == "f32" else 1e-2     # the activations' type
+    for g, r in ((got, ref), (pre, rpre)):
+        g, r = g.reshape(B, M).astype(np.float64), r.reshape(B, M).astype(np.float64)
+        assert np.abs(g - r).max() <= tol * np.abs(r).max()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "int8"])
+def test_batch_special_values(dev, dtype):
+    """Infinities, NaNs, subnormal and huge activations: each token of a batch as that token
+    alone (the vector units' path), NaN for NaN, infinity for infinity, and within the bound."""
+    import torch
+    B, M, K = 8, 48, 256
+    d, h = _make(dtype, B, M, K, seed=5)
+    x = d["x"].reshape(B, K).clone()
+    x[1, 3], x[2, 200], x[3, 17] = float("inf"), float("nan"), float("-inf")
+    x[3, 18] = float("inf")
+    x[4] *= 1e-39          # subnormal activations
+    x[5] *= 1e35
+    x[6] = 0
+    d = dict(d, x=x)
+    whole, _ = _run(d, dtype, B, M, K, False, False, out_dtype="f32")
+    whole = whole.reshape(B, M)
+    h = dict(h, x=x.float().numpy())
+    for b in range(B):
+        one, _ = _run(dict(d, x=x[b].contiguous()), dtype, 1, M, K, False, False, out_dtype="f32")
+        assert np.array_equal(np.isnan(one), np.isnan(whole[b])), b
+        inf = np.isinf(one)
+        assert np.array_equal(one[inf], whole[b][inf]), b
+        if b not in (1, 2, 3):
+            bound = 2 * _bound(dict(h, x=h["x"][b]), 1, M, K)[0]
+            assert np.all(np.abs(one.astype(np.float64) - whole[b]) <= bound), b
+
+
+@pytest.mark.parametrize("dtype,kv", [("f32", "f32"), ("bf16", "bf16"), ("int8", "bf16"), ("bf16", "int8"),
+                                      ("bf16", "fp8"), ("int8", "int8"), ("fp8", "fp8")])
+@pytest.mark.parametrize("B,NH", [(9, 5), (16, 12), (33, 3)])
+def test_batch_qkv_append_equals_gemv_then_append(dev, dtype, kv, B, NH):
+    """qkv, cache bytes and row scales bit for bit, with per-sequence lengths (one beyond maxT)."""
+    import torch
+    kvattn = _kv()
+    HS, K, maxT = 64, 16 * 21, 40
+    M = 3 * NH * HS
+    d, _ = _make(dtype, B, M, K, seed=B + NH)
+    W, x, bias = d["W"].to(dev), d["x"].to(dev).contiguous(), d["bias"].to(dev)
+    scale = None if d.get("scale") is None else d["scale"].to(dev)
+    act = torch.float32 if dtype == "f32" else torch.bfloat16
+    w8 = kv in ("int8", "fp8")
+    n = 2 * B * NH * maxT
+    cache = torch.zeros(n * HS, dtype=torch.uint8 if w8 else act, device=dev)
+    ks_a, ks_b = (torch.zeros(n, device=dev) if w8 else None for _ in range(2))
+    nws = kvattn.gemv_qkv_append_workspace_bytes(B, NH)
+    ws = torch.zeros(nws, dtype=torch.uint8, device=dev)
+    cur = torch.tensor([(7 * b) % maxT for b in range(B - 1)] + [maxT + 5], dtype=torch.int32, device=dev)
+    c_a, c_b = cache.clone(), cache.clone()
+    q_a, q_b = (torch.empty(B * M, dtype=act, device=dev) for _ in range(2))
+    kvattn.gemv(q_a, W, x, B, M, K, w_dtype=dtype, w_scale=scale, bias=bias)
+    kvattn.kv_cache_write(c_a, q_a, B, NH, HS, maxT, kv_dtype=kv, kv_scale=ks_a, cur_len=cur, lens_per_seq=True)
+    kvattn.gemv_qkv_append(q_b, W, x, B, NH, HS, K, c_b, maxT, w_dtype=dtype, kv_dtype=kv, w_scale=scale, bias=bias,
+                           kv_scale=ks_b, cur_len=cur, lens_per_seq=True, workspace=ws, workspace_nbytes=nws)
+    torch.cuda.synchronize()
+    assert torch.equal(q_a.view(torch.uint8), q_b.view(torch.uint8))
+    assert torch.equal(c_a.view(torch.uint8), c_b.view(torch.uint8))
+    if w8:
+        assert torch.equal(ks_a.view(torch.int32), ks_b.view(torch.int32))
+    assert c_b.view(torch.uint8).any()
