@@ -9,8 +9,9 @@
 // 8-bit codes, which are exact in bf16; four 16x16x4 for FP32).  Products are exact and sums FP32,
 // as on the vector units.
 //
-// What bounds it: at the per-layer sizes (0.6 to 9.4 MB of weights) launch and the first memory
-// round trip, so K is split over 4 or 8 waves until one block of loads per wave covers it, and
+// What bounds it: at the per-layer sizes (0.6 to 4.7 MB of BF16 weights) launch and the first memory
+// round trip (768 x 768, 16 tokens: 3.0 us, of 2.0 for an almost empty launch; 10.5 on the vector
+// units), so K is split over 4 or 8 waves until one block of loads per wave covers it, and
 // tiles stay 16 x 16 for the most workgroups.
 //
 // How the operands are read: lane 16 g + r of an MFMA operand holds 16 bytes of row r at K chunk
@@ -20,6 +21,9 @@
 // So a load takes row lane / 4, chunk lane % 4, and ds_bpermute moves the four dwords to the
 // operand's lane.
 #include "fc.hpp"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -244,16 +248,255 @@ __global__ __launch_bounds__(kGemmMaxWaves * kWave) void gemm_kernel(
     }
 }
 
-template <int WT>
-const void* gemm_ptr(bool out_f32, int epi) {
-    constexpr bool kAct = WFmt<WT>::kActF32;
-    if (epi == kEpiAppend) return (const void*)&gemm_kernel<WT, 16, kGemmSteps, kAct, kEpiAppend>;
-    if (epi == kEpiAppend8) {
-        if constexpr (kAct) return nullptr;   // 8-bit caches sit behind bf16 activations
-        else return (const void*)&gemm_kernel<WT, kHd, kGemmSteps, false, kEpiAppend8>;
+__device__ __forceinline__ U32x4 ld16_nt(const uint8_t* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const U32x4*>(p));
+}
+
+// Streamed weights: 16 rows x 128 bytes, two steps, in two loads of whole 128-byte lines (rows 0-7
+// and 8-15; the wave's low half the first 64 bytes of each, its high half the others).  Swapping
+// the halves between the two registers leaves each step's 16 rows x 64 bytes in one of them.
+__device__ __forceinline__ void unpair(U32x4& a, U32x4& b) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const auto p = __builtin_amdgcn_permlane32_swap(a[e], b[e], false, false);
+        a[e] = p[0];
+        b[e] = p[1];
     }
-    return out_f32 ? (const void*)&gemm_kernel<WT, 16, kGemmSteps, true, kEpiNone>
-                   : (const void*)&gemm_kernel<WT, 16, kGemmSteps, false, kEpiNone>;
+}
+
+// Tall matrices (a vocabulary table) for more tokens: with 16 x 16 tiles every workgroup reads its
+// tokens from L2 for its 16 rows alone (50304 x 768, 64 tokens: 309 MB of tokens for 77 MB of BF16
+// weights), and each further tile of tokens reads the weights again.  Here a workgroup, one per
+// CU, keeps its 16 NT tokens in LDS for their whole length, in operand order (a step's 64 lanes
+// side by side), and each of its waves takes whole rows, 16 at a time, with no sum across waves.
+// The weights are read once, non-temporally; two blocks of kTallSteps steps are in flight per
+// wave, across row tiles.  50304 x 768, 64 tokens, BF16: 22.7 us (90 MB: 4.0 TB/s; 270 us on the
+// vector units).  What is left above HBM's time is filling LDS before the first product
+// and the 16 waves' common start and end: a CU has 12 or 13 row tiles, so a wave has one.
+// (Two row tiles per wave, 8 waves: 24.8 to 27.9 us; two smaller workgroups per CU: 28.7.)
+constexpr int kTallSteps = 4;
+constexpr int kTallStage = 8;    // 16-byte token loads in flight per lane while LDS is filled
+constexpr int kTallWaves = 16;
+constexpr int kTallRows = 20000;           // from this many rows on (gemm_plan)
+constexpr int kTallGroups = 256;           // workgroups: one per CU
+constexpr long long kTallLds = 144 * 1024;
+// LDS of NT token tiles.
+template <int WT> constexpr long long tall_lds(int K, int NT) {
+    return ((long long)K * WFmt<WT>::kWBytes / 16 + 3) / 4 * NT * kWave * WFmt<WT>::kXBytes;
+}
+
+template <bool kOutF32>
+__device__ __forceinline__ void store_res4(void* p, size_t i, const float (&v)[4]) {
+    if constexpr (kOutF32) {
+        *reinterpret_cast<F32x4*>(reinterpret_cast<float*>(p) + i) = F32x4{v[0], v[1], v[2], v[3]};
+    } else {
+        typedef uint32_t U32x2 __attribute__((ext_vector_type(2)));
+        *reinterpret_cast<U32x2*>(reinterpret_cast<uint16_t*>(p) + i) =
+            U32x2{f32_to_bf16(v[0]) | (uint32_t)f32_to_bf16(v[1]) << 16,
+                  f32_to_bf16(v[2]) | (uint32_t)f32_to_bf16(v[3]) << 16};
+    }
+}
+
+template <int WT, int NT, bool kOutF32>
+__global__ __launch_bounds__(kTallWaves * kWave) void gemm_tall_kernel(
+    const uint8_t* pk_W, const uint8_t* pk_x, const float* pk_w_scale, const void* pk_bias, int pk_M, int pk_K,
+    int pk_B, int pk_col_tiles, int pk_groups, GemvArgs a) {
+    using F = WFmt<WT>;
+    constexpr int kT = kTallSteps, kW = kTallWaves, kRows = 16;
+    constexpr int kXP = F::kXBytes / 16, kPieces = kTallStage / kXP;
+    extern __shared__ U32x4 xs[];           // [steps][NT][kXP][64]
+    const int M = pk_M & kRowMask, K = pk_K, B = pk_B;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int j8 = blockIdx.x >> 3;
+    const int mq = div_uniform(j8, pk_col_tiles);
+    const int grp = mq * 8 + (blockIdx.x & 7), b0 = (j8 - mq * pk_col_tiles) * 16 * NT;
+    if (grp >= pk_groups) return;
+    const int nch = K * F::kWBytes / 16;
+    const int nsteps = (nch + 3) / 4, nblk = (nsteps + kT - 1) / kT;
+    const int src = (((lane & 15) << 2) | (lane >> 4)) * 4;
+    const int lr = lane >> 2, lc = lane & 3;
+    // This workgroup's row tiles, [tile0, tile1).
+    const int tiles = (M + kRows - 1) / kRows;
+    const int tile0 = (int)((long long)tiles * grp / pk_groups), tile1 = (int)((long long)tiles * (grp + 1) / pk_groups);
+
+    struct Block { U32x4 w[kT]; };
+    auto load = [&](Block& t, int tile, int blk) {
+        const int r0 = tile * kRows + (lr & 7);
+        const uint8_t* p0 = pk_W + (size_t)min(r0, M - 1) * K * F::kWBytes;
+        const uint8_t* p1 = pk_W + (size_t)min(r0 + 8, M - 1) * K * F::kWBytes;
+#pragma unroll
+        for (int u = 0; u < kT; u += 2) {
+            const uint32_t c = (uint32_t)min((blk * kT + u) * 4 + 4 * (lane >> 5) + lc, nch - 1) * 16u;
+            t.w[u] = ld16_nt(p0 + c);
+            t.w[u + 1] = ld16_nt(p1 + c);
+        }
+    };
+    Block wa, wb;
+    int tile = tile0 + wave, blk = 0;       // what is consumed next
+    int ltile = tile, lblk = 0;             // what is loaded next
+    auto next = [&](Block& t) {
+        if (ltile >= tile1) return false;
+        load(t, ltile, lblk);
+        if (++lblk == nblk) { lblk = 0; ltile += kW; }
+        return true;
+    };
+    const bool busy = next(wa);
+    bool more = next(wb);
+    // Row scales and biases of the tile that is worked on, for the rows this lane stores.
+    float ws[4], bias[4];
+    auto load_rows = [&]() {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int mr = min(tile * kRows + 4 * lc + e, M - 1);
+            ws[e] = F::k8bit ? pk_w_scale[mr] : 1.0f;
+            bias[e] = pk_bias ? load_act<WT>(pk_bias, mr) : 0.0f;
+        }
+    };
+    load_rows();
+    // Tokens to LDS: chunk c of token t of tile j goes to step c / 4, lane 16 (c % 4) + t.
+    const int pieces = nsteps * NT;
+    for (int i0 = wave; i0 < pieces; i0 += kW * kPieces) {
+        U32x4 v[kPieces][kXP];
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) {
+            const int i = min(i0 + k * kW, pieces - 1), st = i / NT, j = i - st * NT;
+            const uint8_t* p = pk_x + (size_t)min(b0 + 16 * j + lr, B - 1) * K * 2 +
+                               (size_t)min(st * 4 + lc, nch - 1) * F::kXBytes;
+#pragma unroll
+            for (int h = 0; h < kXP; ++h) v[k][h] = ld16(p + 16 * h);
+        }
+#pragma unroll
+        for (int k = 0; k < kPieces; ++k) {
+            const int i = i0 + k * kW;
+            if (i >= pieces) break;
+#pragma unroll
+            for (int h = 0; h < kXP; ++h) {
+                if (i / NT * 4 + lc >= nch) v[k][h] = U32x4{0u, 0u, 0u, 0u};
+                xs[(i * kXP + h) * kWave + lane] = from_lane(v[k][h], src);
+            }
+        }
+    }
+    __syncthreads();
+    if (!busy) return;
+
+    // FP32 sums: a block's four steps as a tree, blocks in turn to two sums.
+    F32x4 acc[2][NT];
+    // Four outputs of a token in one store, where they are aligned.
+    const bool vec_ok = (((uintptr_t)a.out | (uintptr_t)a.pre_gelu) & (kOutF32 ? 15u : 7u)) == 0;
+    auto clear = [&]() {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[0][j] = acc[1][j] = F32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    clear();
+    auto consume = [&](Block& t, auto which) {
+        constexpr int q = decltype(which)::value;
+        const int st0 = blk * kT;
+#pragma unroll
+        for (int u = 0; u < kT; u += 2) unpair(t.w[u], t.w[u + 1]);
+        if ((st0 + kT) * 4 > nch) {
+#pragma unroll
+            for (int u = 0; u < kT; ++u)
+                if ((st0 + u) * 4 + lc >= nch) t.w[u] = U32x4{0u, 0u, 0u, 0u};
+        }
+        F32x4 even[NT], pair[NT];
+#pragma unroll
+        for (int u = 0; u < kT; ++u) {
+            const int st = min(st0 + u, nsteps - 1);   // steps beyond the row: zero weights
+            const U32x4 wv = from_lane(t.w[u], src);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                U32x4 xv[kXP];
+#pragma unroll
+                for (int h = 0; h < kXP; ++h) xv[h] = xs[((st * NT + j) * kXP + h) * kWave + lane];
+                const F32x4 v = step_product<WT>(wv, xv);
+                if (u % 2 == 0) even[j] = v;
+                else if (u == 1) pair[j] = even[j] + v;
+                else acc[q][j] += pair[j] + (even[j] + v);
+            }
+        }
+        if (++blk < nblk) return;
+        // The tile is done: lane 16 g + r holds rows 4 g .. 4 g + 3 of token r.  Moved to lane 4 r + g,
+        // four neighbouring lanes store 16 rows of one token.
+        const int m = tile * kRows + 4 * lc, back = (lc * 16 + lr) * 4;
+        const bool whole = M % 4 == 0 && m < M && vec_ok;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const F32x4 sum = acc[0][j] + acc[1][j];
+            const F32x4 v = __builtin_bit_cast(F32x4, from_lane(__builtin_bit_cast(U32x4, sum), back));
+            const int b = b0 + 16 * j + lr;
+            if (b >= B) continue;
+            const size_t o = (size_t)b * M + m;
+            float pre[4], act[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                pre[e] = v[e] * ws[e] + bias[e];
+                act[e] = (pk_M & kGeluFlag) ? gelu_tanh(pre[e]) : pre[e];
+            }
+            if (whole) {
+                if (a.pre_gelu) store_res4<kOutF32>(a.pre_gelu, o, pre);
+                store_res4<kOutF32>(a.out, o, act);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (m + e >= M) break;
+                    if (a.pre_gelu) store_res<kOutF32>(a.pre_gelu, o + e, pre[e]);
+                    store_res<kOutF32>(a.out, o + e, act[e]);
+                }
+            }
+        }
+        clear();
+        blk = 0;
+        tile += kW;
+        load_rows();
+    };
+    while (true) {
+        consume(wa, std::integral_constant<int, 0>{});
+        if (!more) break;
+        more = next(wa);
+        consume(wb, std::integral_constant<int, 1>{});
+        if (!more) break;
+        more = next(wb);
+    }
+}
+
+template <int WT, int NT>
+const void* tall_ptr(bool out_f32) {
+    return out_f32 ? (const void*)&gemm_tall_kernel<WT, NT, true> : (const void*)&gemm_tall_kernel<WT, NT, false>;
+}
+
+// How a call runs on the matrix cores: rows (tall: per wave) and tokens per workgroup.
+struct GemmPlan {
+    const void* fn;
+    int rows, cols;
+    bool tall;
+};
+
+// fn == nullptr: no kernel for this call.
+template <int WT>
+GemmPlan gemm_plan(int B, int M, int K, bool out_f32, int epi) {
+    constexpr bool kAct = WFmt<WT>::kActF32;
+    if (epi == kEpiAppend8) {
+        if constexpr (kAct) return {};   // 8-bit caches sit behind bf16 activations
+        else return {(const void*)&gemm_kernel<WT, kHd, kGemmSteps, false, kEpiAppend8>, kHd, 16, false};
+    }
+    if (epi == kEpiAppend) return {(const void*)&gemm_kernel<WT, 16, kGemmSteps, kAct, kEpiAppend>, 16, 16, false};
+    // Tall matrices whose tokens fit in LDS together (us per call, 16 x 16 tiles / tokens in LDS):
+    //   50304 x 768   BF16  8: 18.8 / 17.4   16: 21.7 / 17.6   32: 31.9 / 19.0   64: 49.6 / 22.7
+    //                 INT8                   16: 10.4 / 12.6   32: 16.2 / 14.9   64: 27.9 / 21.1
+    //   24000 x 1024  BF16  32: 23.8 / 14.5  INT8  32: 13.7 / 11.8
+    //   16384 x 768   BF16  32:  9.3 / 10.1  INT8  32:  7.7 /  8.6   64: 11.9 / 13.5
+    // FP32 weights gain nothing (24000 x 1024, 64: 66.7 / 73.4).
+    if constexpr (!kAct) {
+        const int nt = B <= 16 ? 1 : (B <= 32 ? 2 : 4);
+        if (M >= kTallRows && B > (WT == KVATTN_KV_BF16 ? 8 : 16) && tall_lds<WT>(K, nt) <= kTallLds) {
+            if (nt == 4) return {tall_ptr<WT, 4>(out_f32), 16, 64, true};
+            if (nt == 2) return {tall_ptr<WT, 2>(out_f32), 16, 32, true};
+            if constexpr (WT == KVATTN_KV_BF16) return {tall_ptr<WT, 1>(out_f32), 16, 16, true};
+        }
+    }
+    return {out_f32 ? (const void*)&gemm_kernel<WT, 16, kGemmSteps, true, kEpiNone>
+                    : (const void*)&gemm_kernel<WT, 16, kGemmSteps, false, kEpiNone>, 16, 16, false};
 }
 
 }  // namespace
@@ -272,38 +515,49 @@ namespace kvattn_internal {
 // where a row is long but still one block of gemv.hip.
 bool gemm_takes(int w_dtype, int B, int M, int K) {
     const int from = w_dtype != KVATTN_KV_F32 ? 3 : (K > 1600 && K <= 4096 ? 8 : 4);
-    if (B < from || M >= 8192 || K > (1 << 20)) return false;
-    // Tall matrices stay with gemv.hip; so do grids beyond 2^31 threads.
+    if (B < from || K > (1 << 20)) return false;
+    // Grids beyond 2^31 threads stay with gemv.hip.
     const long long groups = 8ll * ((M + 127) / 128) * ((B + 15) / 16);
     return groups * kGemmMaxWaves * kWave < (1ll << 31);
 }
 
 // The launch for arguments that launch_gemv has checked.  The waves split a row's steps alike
-// whatever the epilogue, so that the QKV projection with the append in its epilogue sums as the
-// plain one does, bit for bit.
+// whatever the epilogue, so that up to kTallRows rows the QKV projection with the append in its
+// epilogue sums as the plain one does, bit for bit.
 int launch_gemm(GemvArgs a, int w_dtype, bool out_f32, int epi, void* stream) {
     const int wbytes = w_dtype == KVATTN_KV_F32 ? 4 : (w_dtype == KVATTN_KV_BF16 ? 2 : 1);
-    constexpr int cols = 16;
-    int col_tiles = (a.B + cols - 1) / cols;
-    const int rows = epi == kEpiAppend8 ? kHd : 16;
-    const void* fn = nullptr;
+    GemmPlan p;
     switch (w_dtype) {
-        case KVATTN_KV_F32: fn = gemm_ptr<KVATTN_KV_F32>(out_f32, epi); break;
-        case KVATTN_KV_BF16: fn = gemm_ptr<KVATTN_KV_BF16>(out_f32, epi); break;
-        case KVATTN_KV_INT8: fn = gemm_ptr<KVATTN_KV_INT8>(out_f32, epi); break;
-        default: fn = gemm_ptr<KVATTN_KV_FP8_E4M3>(out_f32, epi); break;
+        case KVATTN_KV_F32: p = gemm_plan<KVATTN_KV_F32>(a.B, a.M, a.K, out_f32, epi); break;
+        case KVATTN_KV_BF16: p = gemm_plan<KVATTN_KV_BF16>(a.B, a.M, a.K, out_f32, epi); break;
+        case KVATTN_KV_INT8: p = gemm_plan<KVATTN_KV_INT8>(a.B, a.M, a.K, out_f32, epi); break;
+        default: p = gemm_plan<KVATTN_KV_FP8_E4M3>(a.B, a.M, a.K, out_f32, epi); break;
     }
-    if (!fn) return KVATTN_ERR_DTYPE;
+    if (!p.fn) return KVATTN_ERR_DTYPE;
     const int steps = (a.K * wbytes / 16 + 3) / 4;
-    const int waves = steps <= kGemmSteps * kGemmMinWaves ? kGemmMinWaves : kGemmMaxWaves;
-    int pk_steps = (steps / waves) << 8 | (steps % waves);
-    const long long row_tiles = (a.M + rows - 1) / rows;
-    const long long groups = 8 * ((row_tiles + 7) / 8) * col_tiles;
+    int col_tiles = (a.B + p.cols - 1) / p.cols;
     int pk_m = a.M | (a.gelu ? kGeluFlag : 0);
-    const size_t lds = (size_t)waves * cols * (rows + 4) * sizeof(float);
-    void* params[] = {&a.W, &a.x, &a.w_scale, &a.bias, &pk_m, &a.K, &a.B, &col_tiles, &pk_steps, &a};
-    const hipError_t e = hipLaunchKernel(fn, dim3((unsigned)groups), dim3(waves * kWave), params, lds,
-                                         (hipStream_t)stream);
+    int groups = (a.M + p.rows - 1) / p.rows, waves, last;
+    size_t lds;
+    if (p.tall) {
+        waves = kTallWaves;
+        last = groups = std::min(groups, kTallGroups);
+        lds = (size_t)steps * (p.cols / 16) * kWave * (wbytes == 1 ? 32 : 16);
+        if (lds > 64 * 1024) {
+            const hipError_t e = hipFuncSetAttribute(p.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTallLds);
+            if (e != hipSuccess) {
+                set_last_hip_error((int)e);
+                return KVATTN_ERR_HIP;
+            }
+        }
+    } else {
+        waves = steps <= kGemmSteps * kGemmMinWaves ? kGemmMinWaves : kGemmMaxWaves;
+        last = (steps / waves) << 8 | (steps % waves);
+        lds = (size_t)waves * p.cols * (p.rows + 4) * sizeof(float);
+    }
+    void* params[] = {&a.W, &a.x, &a.w_scale, &a.bias, &pk_m, &a.K, &a.B, &col_tiles, &last, &a};
+    const hipError_t e = hipLaunchKernel(p.fn, dim3(8u * (unsigned)((groups + 7) / 8) * (unsigned)col_tiles),
+                                         dim3(waves * kWave), params, lds, (hipStream_t)stream);
     if (e != hipSuccess) {
         set_last_hip_error((int)e);
         return KVATTN_ERR_HIP;

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle
-from tests.test_gpu_gemv import _kv, _make, _run
+from test_gpu_gemv import _kv, _make, _run
 
 pytestmark = pytest.mark.gpu
 
@@ -47,6 +47,44 @@ def test_batch_against_float64(dev, dtype, B, M, K):
     got, _ = _run(d, dtype, B, M, K, False, False, out_dtype="f32")
     err = np.abs(got.reshape(B, M).astype(np.float64) - _exact(h, B, M, K))
     assert np.all(err <= _bound(h, B, M, K)), float((err / _bound(h, B, M, K)).max())
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "int8", "fp8"])
+@pytest.mark.parametrize("B,M,K", [(9, 20000, 32), (17, 20001, 144), (33, 20015, 272), (64, 20017, 528),
+                                   (70, 24571, 64), (16, 65537, 48)])
+def test_tall_batch_against_float64(dev, dtype, B, M, K):
+    """From 20000 rows on the tokens sit in LDS: 16, 32 or 64 of them, rows in whole and partial
+    tiles of 16 and in several tiles per wave (65537 rows), M not a multiple of 4, K of a partial
+    block of steps, and tokens beyond one workgroup's."""
+    d, h = _make(dtype, B, M, K, seed=B + M + K)
+    d = dict(d, W=_guarded(d["W"]), x=_guarded(d["x"]))
+    got, _ = _run(d, dtype, B, M, K, False, False, out_dtype="f32")
+    bound = _bound(h, B, M, K)
+    err = np.abs(got.reshape(B, M).astype(np.float64) - _exact(h, B, M, K))
+    assert np.all(err <= bound), float((err / bound).max())
+
+
+@pytest.mark.parametrize("out_dtype", ["f32", "bf16"])
+def test_tall_batch_gelu_and_unaligned_outputs(dev, out_dtype):
+    """GELU and pre_gelu from the kernel with tokens in LDS, into outputs that vector stores fit and
+    into ones a single element further on: the same values."""
+    import torch
+    kvattn = _kv()
+    B, M, K = 20, 20480, 96
+    d, h = _make("bf16", B, M, K, seed=9)
+    odt = torch.float32 if out_dtype == "f32" else torch.bfloat16
+    dd = {k: v.to(dev) for k, v in d.items() if v is not None}
+    got = []
+    for shift in (0, 1):
+        out, pre = (torch.full((B * M + 1,), float("nan"), dtype=odt, device=dev)[shift:shift + B * M] for _ in range(2))
+        kvattn.gemv(out, dd["W"], dd["x"], B, M, K, w_dtype="bf16", bias=dd["bias"], pre_gelu=pre, gelu=True,
+                    out_dtype=out_dtype)
+        got.append((out.float().cpu().numpy(), pre.float().cpu().numpy()))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    ref, rpre = oracle.gemv(h["W"], h["x"], B, M, K, bias=h["bias"], gelu=True, want_pre=True)
+    tol = 1e-5 if out_dtype == "f32" else 1e-2
+    for g, r in ((got[0][0], ref), (got[0][1], rpre)):
+        assert np.abs(g - r.reshape(-1)).max() <= tol * np.abs(r).max()
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "int8", "fp8"])
@@ -120,3 +158,25 @@ def test_batch_qkv_append_equals_gemv_then_append(dev, dtype, kv, B, NH):
     if w8:
         assert torch.equal(ks_a.view(torch.int32), ks_b.view(torch.int32))
     assert c_b.view(torch.uint8).any()
+
+
+def test_tall_batch_in_a_graph(dev):
+    """The kernel with tokens in LDS (more than 64 KB of it) captured and replayed over new tokens,
+    with eager work in between: every replay as the eager call."""
+    import torch
+    kvattn = _kv()
+    B, M, K = 64, 20000, 768
+    d, _ = _make("bf16", B, M, K, seed=3, with_bias=False)
+    W, x = d["W"].to(dev), d["x"].to(dev).reshape(B, K).contiguous()
+    out, ref = (torch.empty(B, M, device=dev) for _ in range(2))
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g):
+        kvattn.gemv(out, W, x, B, M, K, w_dtype="bf16", out_dtype="f32")
+    for rep in range(3):
+        x.copy_(x.roll(rep + 1, dims=0))
+        kvattn.gemv(ref, W, x, B, M, K, w_dtype="bf16", out_dtype="f32")
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), rep
