@@ -80,6 +80,11 @@ __device__ __forceinline__ float dpp(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kCtrl, 0xF, 0xF, true));
 }
 
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, 0xF, 0xF, true);
+}
+
 // Sum over the kLanes lanes holding one row (aligned groups of 4, 8 or 16 lanes).
 template <int kLanes>
 __device__ __forceinline__ float row_sum(float x) {
