@@ -155,10 +155,25 @@ def _ptr(x) -> Optional[int]:
     return x.data_ptr()
 
 
+# The handle of torch's current stream on the current device.  torch.cuda.current_stream() builds
+# a Stream object for it, 2.8 us of an eager call's 8.3 us; the handle alone takes 0.1 us.
+_current_stream = None
+
+
+def _find_current_stream():
+    import torch
+    raw, device = getattr(torch._C, "_cuda_getCurrentRawStream", None), torch.cuda.current_device
+    if raw is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: raw(device())
+
+
 def _stream(stream) -> Optional[int]:
     if stream is None:
-        import torch
-        return torch.cuda.current_stream().cuda_stream
+        global _current_stream
+        if _current_stream is None:
+            _current_stream = _find_current_stream()
+        return _current_stream()
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
