@@ -398,7 +398,7 @@ struct Tile {
 // slot's maxT, and at least 1), so no load sits behind a branch and all of them issue back
 // to back.  Those rows hold another row's data: consume_tile<kChecked>, and fused_single's
 // one-tile path, mask them by selection (score -inf, V chunk and V scale zero).
-template <int DT, int U, bool kChecked>
+template <int DT, int U, bool kChecked, bool kNt>
 __device__ __forceinline__ void load_tile(Tile<DT, U>& t, const Slot& sl, int r, int r1, int slot_row) {
     using R = Row<DT>;
     constexpr int kRPL = kRowsPerLoad<DT>;
@@ -406,8 +406,8 @@ __device__ __forceinline__ void load_tile(Tile<DT, U>& t, const Slot& sl, int r,
     for (int u = 0; u < U; ++u) {
         int row = r + u * kRPL + slot_row;
         if (kChecked) row = max(min(row, r1 - 1), 0);
-        t.k[u] = load16(sl.k + (uint32_t)row * R::kBytes);
-        t.v[u] = load16(sl.v + (uint32_t)row * R::kBytes);
+        t.k[u] = load16<kNt>(sl.k + (uint32_t)row * R::kBytes);
+        t.v[u] = load16<kNt>(sl.v + (uint32_t)row * R::kBytes);
         if constexpr (R::k8bit) { t.ks[u] = sl.ks[row]; t.vs[u] = sl.vs[row]; }
     }
     // INT8 full tiles (the walk past a segment's first tile): keep every load of the tile
@@ -493,7 +493,7 @@ __device__ __forceinline__ void consume_tile(const Tile<DT, U>& t, int r, int r1
 // rows of that tile at or beyond r1 are masked.  The q slice is requested after the tile's
 // K/V loads, so nothing that depends on q is scheduled ahead of them.  kFresh: the row
 // `cur` (if inside [r0, r1)) is taken from f instead of the cache.
-template <int DT, int kU, bool kFresh, bool kHw = false>
+template <int DT, int kU, bool kFresh, bool kHw, bool kNt>
 __device__ __forceinline__ void online_rows_from(Tile<DT, kU>& t0, const QRaw<DT>& qr,
                                                  const Slot& sl, int r0, int r1, int slot_row, float qscale,
                                                  const FreshRaw<DT>& fr, const FreshDst& fd, int cur,
@@ -509,12 +509,12 @@ __device__ __forceinline__ void online_rows_from(Tile<DT, kU>& t0, const QRaw<DT
     Tile<DT, kU> t;
     int r = r0 + kTile;
     for (; r + kTile <= r1; r += kTile) {
-        load_tile<DT, kU, false>(t, sl, r, r1, slot_row);
+        load_tile<DT, kU, false, kNt>(t, sl, r, r1, slot_row);
         if (holds(r)) patch_tile<DT, kU>(t, fr, fd, r, slot_row, cur);
         consume_tile<DT, kU, false, kHw>(t, r, r1, slot_row, q, m, l, acc);
     }
     if (r < r1) {
-        load_tile<DT, kU, true>(t, sl, r, r1, slot_row);
+        load_tile<DT, kU, true, kNt>(t, sl, r, r1, slot_row);
         if (holds(r)) patch_tile<DT, kU>(t, fr, fd, r, slot_row, cur);
         consume_tile<DT, kU, true, kHw>(t, r, r1, slot_row, q, m, l, acc);
     }
@@ -590,8 +590,8 @@ __device__ __forceinline__ void online_tiles_paged(const PagedView& pv, int b, i
         const int a0 = ra / P * P, b0 = rb / P * P;
         auto ld = [&](Tile<DT, kU>& tt, int page, int rr, int p0) {
             const Slot sp = page_slot<DT>(pv, page, h, slice);
-            if (rr + kTile <= j1) load_tile<DT, kU, false>(tt, sp, rr - p0, j1 - p0, slot_row);
-            else load_tile<DT, kU, true>(tt, sp, rr - p0, j1 - p0, slot_row);
+            if (rr + kTile <= j1) load_tile<DT, kU, false, true>(tt, sp, rr - p0, j1 - p0, slot_row);
+            else load_tile<DT, kU, true, true>(tt, sp, rr - p0, j1 - p0, slot_row);
         };
         if (va) ld(t, pa, ra, a0);
         if (vb) ld(t1, pb, rb, b0);
@@ -624,11 +624,11 @@ __device__ __forceinline__ void online_tiles_paged(const PagedView& pv, int b, i
         // Full tiles take the unchecked loads and scores (no per-row conditions around the
         // loads), as the contiguous walk does; only a segment's last tile is checked.
         if (r + kTile <= j1) {
-            load_tile<DT, kU, false>(t, sp, r - pr0, j1 - pr0, slot_row);
+            load_tile<DT, kU, false, true>(t, sp, r - pr0, j1 - pr0, slot_row);
             fresh();
             consume_tile<DT, kU, false, kHw>(t, r - pr0, j1 - pr0, slot_row, q, m, l, acc);
         } else {
-            load_tile<DT, kU, true>(t, sp, r - pr0, j1 - pr0, slot_row);
+            load_tile<DT, kU, true, true>(t, sp, r - pr0, j1 - pr0, slot_row);
             fresh();
             consume_tile<DT, kU, true, kHw>(t, r - pr0, j1 - pr0, slot_row, q, m, l, acc);
         }
@@ -639,7 +639,7 @@ __device__ __forceinline__ void online_tiles_paged(const PagedView& pv, int b, i
 // fused_single: one workgroup per (b,h), grid B*NH.  Pass 1 writes every score to LDS
 // and finds the exact maximum; pass 2 weights V with exp2(score - max).
 // ------------------------------------------------------------------------------------
-template <int DT, int U, bool kChecked, bool kFresh, bool kHw = false>
+template <int DT, int U, bool kChecked, bool kFresh, bool kHw, bool kNt>
 __device__ __forceinline__ void score_tile(const Slot& sl, int r, int total, int slot_row, int slice,
                                            const float (&q)[Row<DT>::kElems], float* scores, float& mloc,
                                            const FreshRaw<DT>& fr, const FreshDst& fd) {
@@ -651,7 +651,7 @@ __device__ __forceinline__ void score_tile(const Slot& sl, int r, int total, int
     for (int u = 0; u < U; ++u) {
         const int row = r + u * kRPL + slot_row;
         if (!kChecked || row < total) {
-            kd[u] = load16(sl.k + (uint32_t)row * R::kBytes);
+            kd[u] = load16<kNt>(sl.k + (uint32_t)row * R::kBytes);
             if constexpr (R::k8bit) ks[u] = sl.ks[row];
         } else {
             kd[u] = make_uint4(0u, 0u, 0u, 0u);
@@ -683,7 +683,7 @@ __device__ __forceinline__ void score_tile(const Slot& sl, int r, int total, int
     }
 }
 
-template <int DT, int U, bool kChecked, bool kFresh>
+template <int DT, int U, bool kChecked, bool kFresh, bool kNt>
 __device__ __forceinline__ void weight_tile(const Slot& sl, int r, int total, int slot_row, float M,
                                             const float* scores, float& l, float (&acc)[Row<DT>::kElems],
                                             const FreshRaw<DT>& fr) {
@@ -695,7 +695,7 @@ __device__ __forceinline__ void weight_tile(const Slot& sl, int r, int total, in
     for (int u = 0; u < U; ++u) {
         const int row = r + u * kRPL + slot_row;
         if (!kChecked || row < total) {
-            vd[u] = load16(sl.v + (uint32_t)row * R::kBytes);
+            vd[u] = load16<kNt>(sl.v + (uint32_t)row * R::kBytes);
             if constexpr (R::k8bit) vs[u] = sl.vs[row];
         } else {
             vd[u] = make_uint4(0u, 0u, 0u, 0u);
@@ -730,7 +730,7 @@ __device__ __forceinline__ void weight_tile(const Slot& sl, int r, int total, in
 
 // kFresh: append and attend in one launch; kv_out / kv_scale_out receive the current
 // token's row (they alias kv / kv_scale, whose row cur_len is then never used).
-template <int DT, int kThreads, int kU, bool kFresh>
+template <int DT, int kThreads, int kU, bool kFresh, bool kNt>
 // Parameters in the order the first loads need them: the leading 14 dwords are preloaded
 // into SGPRs at wave launch (the library is built with kernel-argument preloading).
 __global__ __launch_bounds__(kThreads) void fused_single_kernel(
@@ -758,7 +758,7 @@ __global__ __launch_bounds__(kThreads) void fused_single_kernel(
     Tile<DT, kU> t;
     QRaw<DT> qr;
     if (spec) {
-        load_tile<DT, kU, true>(t, sl, wave * kTile, spec_lim, slot_row);
+        load_tile<DT, kU, true, kNt>(t, sl, wave * kTile, spec_lim, slot_row);
         qr = load_q<DT>(qkv, b, h, NH, slice);
     }
     FreshRaw<DT> fr{};
@@ -778,7 +778,7 @@ __global__ __launch_bounds__(kThreads) void fused_single_kernel(
         // scores stay in registers and only the workgroup maximum passes through LDS.
         const int r = wave * kTile;
         if (!spec || total > spec_lim) {
-            load_tile<DT, kU, true>(t, sl, r, total, slot_row);
+            load_tile<DT, kU, true, kNt>(t, sl, r, total, slot_row);
             qr = load_q<DT>(qkv, b, h, NH, slice);
         }
         convert_q<DT, true>(qr, qscale, q);
@@ -817,9 +817,9 @@ __global__ __launch_bounds__(kThreads) void fused_single_kernel(
         float mloc = kStartMax;
         const int full = total / kTile * kTile;
         for (int r = wave * kTile; r < full; r += kW * kTile)
-            score_tile<DT, kU, false, kFresh, true>(sl, r, total, slot_row, slice, q, s_scores, mloc, fr, fd);
+            score_tile<DT, kU, false, kFresh, true, kNt>(sl, r, total, slot_row, slice, q, s_scores, mloc, fr, fd);
         for (int r = full + wave * kTile; r < total; r += kW * kTile)
-            score_tile<DT, kU, true, kFresh, true>(sl, r, total, slot_row, slice, q, s_scores, mloc, fr, fd);
+            score_tile<DT, kU, true, kFresh, true, kNt>(sl, r, total, slot_row, slice, q, s_scores, mloc, fr, fd);
         mloc = slot_reduce<R::kLanes, true>(mloc);   // a row's lanes hold the same scores
         if (lane == 0) s_max[wave] = mloc;
         __syncthreads();
@@ -828,9 +828,9 @@ __global__ __launch_bounds__(kThreads) void fused_single_kernel(
         for (int w = 1; w < kW; ++w) M = fmaxf(M, s_max[w]);
         // Pass 2: V rows weighted by exp2(score - M).
         for (int r = wave * kTile; r < full; r += kW * kTile)
-            weight_tile<DT, kU, false, kFresh>(sl, r, total, slot_row, M, s_scores, l, acc, fr);
+            weight_tile<DT, kU, false, kFresh, kNt>(sl, r, total, slot_row, M, s_scores, l, acc, fr);
         for (int r = full + wave * kTile; r < total; r += kW * kTile)
-            weight_tile<DT, kU, true, kFresh>(sl, r, total, slot_row, M, s_scores, l, acc, fr);
+            weight_tile<DT, kU, true, kFresh, kNt>(sl, r, total, slot_row, M, s_scores, l, acc, fr);
     }
 
     l = slot_reduce<R::kLanes, false>(l);
@@ -1139,7 +1139,7 @@ __device__ __forceinline__ void merge_partials(void* out, const float* part_out,
 // kFresh: append and attend in one launch (the workgroup whose segment holds position
 // cur_len takes that row from qkv and writes it to the cache).  kPaged: the cache is a page
 // pool addressed through a block table (segments then start at multiples of the tile).
-template <int DT, int kMode, int kW, int kU, bool kFresh, bool kPaged>
+template <int DT, int kMode, int kW, int kU, bool kFresh, bool kPaged, bool kNt>
 __global__ __launch_bounds__(kW * kWave, kW == kWaves ? KVATTN_STREAM_MIN_BLOCKS : 1) void split_kernel(const uint8_t* pk_kv, const void* pk_qkv, const int* pk_len, int pk_NH, int pk_maxT,
                                          int pk_S, int pk_seg_rows, int pk_BNH, int pk_spec, int pk_B, SplitArgs a) {
     // The fields that the first loads depend on also come as leading scalar parameters: the
@@ -1235,7 +1235,7 @@ __global__ __launch_bounds__(kW * kWave, kW == kWaves ? KVATTN_STREAM_MIN_BLOCKS
             g_end = nend;
             g_has_tile = !first || g_w1 <= j0 + nom;
             const Slot sl0 = make_slot<DT>(a.kv, a.kv_scale, 1, BNH, a.maxT, bh0, slice);
-            if (g_has_tile) load_tile<DT, kU, true>(g_tile, sl0, g_w0, g_w1, slot_row);
+            if (g_has_tile) load_tile<DT, kU, true, kNt>(g_tile, sl0, g_w0, g_w1, slot_row);
             // The sequence index (a division by NH) is needed only for q's address: keep it
             // behind the tile's requests.
             __builtin_amdgcn_sched_barrier(0);
@@ -1327,22 +1327,22 @@ __global__ __launch_bounds__(kW * kWave, kW == kWaves ? KVATTN_STREAM_MIN_BLOCKS
                             x1 = min(x0 + kTileRows, j1);
                         }
                         w1 = min(w1, j1);
-                        if (kDev && !spec_tile && w0 < w1) load_tile<DT, kU, true>(t0, sl, w0, w1, slot_row);
-                        if (kDev && x0 < x1) load_tile<DT, kU, true>(tx, sl, x0, x1, slot_row);
+                        if (kDev && !spec_tile && w0 < w1) load_tile<DT, kU, true, kNt>(t0, sl, w0, w1, slot_row);
+                        if (kDev && x0 < x1) load_tile<DT, kU, true, kNt>(tx, sl, x0, x1, slot_row);
                     } else {
                         const int per_wave = ceil_div_i(j1 - j0, kW);
                         w0 = min(j0 + wave * per_wave, j1);
                         w1 = min(w0 + per_wave, j1);
-                        load_tile<DT, kU, true>(t0, sl, w0, w1, slot_row);
+                        load_tile<DT, kU, true, kNt>(t0, sl, w0, w1, slot_row);
                         q0 = load_q<DT>(a.qkv, it.b, it.h, a.NH, slice);
                         if constexpr (kFresh) fr = load_fresh<DT>(a.qkv, it.b, it.h, a.NH, slice);
                     }
                     if constexpr (kFresh)
                         fd = fresh_dst(a.kv_out, a.kv_scale_out, 1, BNH, a.maxT, bh, slice, cur);
-                    online_rows_from<DT, kU, kFresh, kHwDot>(t0, q0, sl, w0, w1, slot_row, a.qscale, fr, fd, cur, m, l,
+                    online_rows_from<DT, kU, kFresh, kHwDot, kNt>(t0, q0, sl, w0, w1, slot_row, a.qscale, fr, fd, cur, m, l,
                                                              acc);
                     if (kDev && x0 < x1)
-                        online_rows_from<DT, kU, kFresh, kHwDot>(tx, q0, sl, x0, x1, slot_row, a.qscale, fr, fd, cur, m,
+                        online_rows_from<DT, kU, kFresh, kHwDot, kNt>(tx, q0, sl, x0, x1, slot_row, a.qscale, fr, fd, cur, m,
                                                                  l, acc);
                 }
                 // A producer's look at its merger's XCD word: requested once its tiles are consumed,
@@ -1512,8 +1512,8 @@ __global__ __launch_bounds__(kW * kWave, kW == kWaves ? KVATTN_STREAM_MIN_BLOCKS
                                                     a.kv_out, a.kv_scale_out, cur, mm, ll, ac);
                                         } else {
                                             Tile<DT, kU> tf;
-                                            load_tile<DT, kU, true>(tf, sl, sj0, sj1, slot_row);
-                                            online_rows_from<DT, kU, kFresh, kHwDot>(tf, q0, sl, sj0, sj1, slot_row,
+                                            load_tile<DT, kU, true, kNt>(tf, sl, sj0, sj1, slot_row);
+                                            online_rows_from<DT, kU, kFresh, kHwDot, kNt>(tf, q0, sl, sj0, sj1, slot_row,
                                                                                      a.qscale, fr, fd, cur, mm, ll, ac);
                                         }
                                     }
@@ -1912,6 +1912,23 @@ int dispatch_dtype(int dt, F&& f) {
     }
 }
 
+// Calls that attend at most this much read K and V with plain loads: too few workgroups to keep
+// the memory system busy, which non-temporal loads slow down.  us per call, non-temporal / plain
+// (12-24 calls per graph, NH = 12, sequences : positions):
+//   fused_single  F32   1:200 4.69 / 3.72   4:200 (10 MB)  4.95 / 3.95   16:200 (39 MB) 6.13 / 6.27
+//                 BF16  4:200 3.73 / 3.26  16:200 (10 MB)  4.45 / 4.23   64:200 (39 MB) 8.57 / 9.00
+//                 INT8  4:200 3.50 / 3.15  16:200          3.83 / 3.63   64:200 (21 MB) 6.45 / 6.59
+//   designated    F32  1:1024 4.79 / 4.32   2:1024 (13 MB) 5.75 / 5.82
+//                 BF16 1:1024 4.25 / 3.86   2:1024         4.56 / 4.29   4:1024 (13 MB) 5.62 / 5.63
+//                 INT8 1:1024 4.04 / 4.06   4:1024         5.11 / 5.14 (left as they are)
+constexpr long long kPlainMaxBytes = 10ll << 20;
+
+// K and V bytes a call attends at most, the host's hint given.
+long long attended_bytes(int B, int NH, int rows, int kv_dtype) {
+    const int row = kv_dtype == KVATTN_KV_F32 ? 512 : (kv_dtype == KVATTN_KV_BF16 ? 256 : 136);
+    return (long long)B * NH * rows * row;
+}
+
 // kv_out == nullptr: attention only.  Otherwise the kernel also appends the current
 // token's row into kv_out / kv_scale_out (the same cache as kv / kv_scale).
 // spec_rows: the hinted length the kernel may request tiles for before it reads the device
@@ -1923,21 +1940,27 @@ int launch_fused_single(void* out, const void* qkv, const void* kv, const float*
     const size_t lds = (size_t)maxT * sizeof(float);
     if (lds > kFusedMaxLds) return KVATTN_ERR_LDS;
     const float qs = qscale_for(kHeadDim);
+    const bool plain = attended_bytes(B, NH, hint_rows > 0 ? hint_rows : maxT, kv_dtype) <= kPlainMaxBytes;
     const bool short_tiles = hint_rows > 0 && hint_rows <= kFusedShortWaves * kFusedShortRows;
     const bool wide_f32 = kv_dtype == KVATTN_KV_F32 && (long long)B * NH > kFusedF32WideHeads;
     return dispatch_dtype(kv_dtype, [&](auto dtc) -> int {
         constexpr int DT = decltype(dtc)::value;
-        auto launch = [&](auto threads_c, auto unroll_c) {
+        auto launch_as = [&](auto threads_c, auto unroll_c, auto nt_c) {
             constexpr int kThreads = decltype(threads_c)::value;
             constexpr int kU = decltype(unroll_c)::value;
+            constexpr bool kNt = decltype(nt_c)::value;
             if (kv_out)
-                hipLaunchKernelGGL((fused_single_kernel<DT, kThreads, kU, true>), dim3(B * NH), dim3(kThreads), lds,
+                hipLaunchKernelGGL((fused_single_kernel<DT, kThreads, kU, true, kNt>), dim3(B * NH), dim3(kThreads), lds,
                                    stream, qkv, (const uint8_t*)kv, cur_len, lens_per_seq, B, NH, maxT, spec_rows, qs,
                                    kv_scale, out, (uint8_t*)kv_out, kv_scale_out);
             else
-                hipLaunchKernelGGL((fused_single_kernel<DT, kThreads, kU, false>), dim3(B * NH), dim3(kThreads), lds,
+                hipLaunchKernelGGL((fused_single_kernel<DT, kThreads, kU, false, kNt>), dim3(B * NH), dim3(kThreads), lds,
                                    stream, qkv, (const uint8_t*)kv, cur_len, lens_per_seq, B, NH, maxT, spec_rows, qs,
                                    kv_scale, out, (uint8_t*)nullptr, (float*)nullptr);
+        };
+        auto launch = [&](auto threads_c, auto unroll_c) {
+            if (plain) launch_as(threads_c, unroll_c, std::false_type{});
+            else launch_as(threads_c, unroll_c, std::true_type{});
         };
         if (short_tiles)
             launch(std::integral_constant<int, kFusedShortWaves * kWave>{},
@@ -1959,16 +1982,16 @@ int launch_fused_single(void* out, const void* qkv, const void* kv, const float*
 // kDesignatedDev instance: their first tile is never requested before the length.)
 template <int DT, int W, int U, bool kFresh, bool kPaged>
 const void* split_ptr_mode(int mode) {
-    if (mode == kPartialsOnly) return (const void*)&split_kernel<DT, kPartialsOnly, W, U, kFresh, kPaged>;
+    if (mode == kPartialsOnly) return (const void*)&split_kernel<DT, kPartialsOnly, W, U, kFresh, kPaged, true>;
     if (mode == kPartialsStrided) {
-        if constexpr (W == kWaves) return (const void*)&split_kernel<DT, kPartialsStrided, W, U, kFresh, kPaged>;
+        if constexpr (W == kWaves) return (const void*)&split_kernel<DT, kPartialsStrided, W, U, kFresh, kPaged, true>;
         else return nullptr;
     }
-    if (mode == kLastBlockMerge) return (const void*)&split_kernel<DT, kLastBlockMerge, W, U, kFresh, kPaged>;
-    if (mode == kDesignated) return (const void*)&split_kernel<DT, kDesignated, W, U, kFresh, kPaged>;
+    if (mode == kLastBlockMerge) return (const void*)&split_kernel<DT, kLastBlockMerge, W, U, kFresh, kPaged, true>;
+    if (mode == kDesignated) return (const void*)&split_kernel<DT, kDesignated, W, U, kFresh, kPaged, true>;
     if constexpr (kPaged) return nullptr;
-    else if (mode == kDesignatedDev) return (const void*)&split_kernel<DT, kDesignatedDev, W, U, kFresh, false>;
-    else return (const void*)&split_kernel<DT, kCoopMerge, W, U, kFresh, false>;
+    else if (mode == kDesignatedDev) return (const void*)&split_kernel<DT, kDesignatedDev, W, U, kFresh, false, true>;
+    else return (const void*)&split_kernel<DT, kCoopMerge, W, U, kFresh, false, true>;
 }
 
 template <int DT, int W, int U>
@@ -1985,9 +2008,25 @@ const void* split_ptr(int mode, bool lat, bool fresh, bool paged) {
 
 int split_threads(bool lat) { return (lat ? kWavesLat : kWaves) * kWave; }
 
+// The plain-load form of a designated instance (the latency shape; F32 and BF16, contiguous).
+template <int DT, bool kFresh>
+const void* split_ptr_plain(int mode) {
+    constexpr int W = kWavesLat, U = kUnrollSplitLat<DT>;
+    return mode == kDesignated ? (const void*)&split_kernel<DT, kDesignated, W, U, kFresh, false, false>
+                               : (const void*)&split_kernel<DT, kDesignatedDev, W, U, kFresh, false, false>;
+}
+
 // The split kernel for these arguments: appending when kv_out is set, paged when table is.
 const void* split_ptr_for(const SplitArgs& a, int kv_dtype, int mode, bool lat) {
     const void* fn = nullptr;
+    // Small designated calls read with plain loads (kPlainMaxBytes).
+    if (lat && !a.table && (mode == kDesignated || mode == kDesignatedDev) && !is_8bit(kv_dtype) &&
+        attended_bytes(a.B, a.NH, a.spec_rows > 0 ? a.spec_rows : a.maxT, kv_dtype) <= kPlainMaxBytes) {
+        const bool fresh = a.kv_out != nullptr;
+        if (kv_dtype == KVATTN_KV_F32)
+            return fresh ? split_ptr_plain<KVATTN_KV_F32, true>(mode) : split_ptr_plain<KVATTN_KV_F32, false>(mode);
+        return fresh ? split_ptr_plain<KVATTN_KV_BF16, true>(mode) : split_ptr_plain<KVATTN_KV_BF16, false>(mode);
+    }
     dispatch_dtype(kv_dtype, [&](auto dtc) -> int {
         fn = split_ptr<decltype(dtc)::value>(mode, lat, a.kv_out != nullptr, a.table != nullptr);
         return KVATTN_OK;
