@@ -11,7 +11,7 @@
 //
 // What bounds it: at the per-layer sizes (0.6 to 4.7 MB of BF16 weights) launch and the first memory
 // round trip (768 x 768, 16 tokens: 3.0 us, of 2.0 for an almost empty launch; 10.5 on the vector
-// units), so K is split over 4 or 8 waves until one block of loads per wave covers it, and
+// units), so K is split over 8 waves until one block of loads per wave covers it, and
 // tiles stay 16 x 16 for the most workgroups.
 //
 // How the operands are read: lane 16 g + r of an MFMA operand holds 16 bytes of row r at K chunk
@@ -101,7 +101,9 @@ __device__ __forceinline__ F32x4 step_product(U32x4 w, const U32x4 (&x)[kXP]) {
     }
 }
 
-constexpr int kGemmMinWaves = 4, kGemmMaxWaves = 8;
+// Waves per workgroup, whatever K: 4 for the 12 steps of a K = 768 row of 8-bit weights cost 1 to 4 %
+// of a whole decode step (INT8, 12 tokens, 4 layers: 101.0 us, 97.8 with 8).
+constexpr int kGemmWaves = 8;
 // Steps per block.  6 instead of 3, or 16 waves for the longest rows, measured within 5 % at 768 x
 // 3072, and 6 lost 7-12 % at 768 x 768.
 constexpr int kGemmSteps = 3;
@@ -112,7 +114,7 @@ constexpr int kGemmSteps = 3;
 // beyond the row load something that exists and is dropped (rows and tokens are not stored,
 // chunks enter as zeros).
 template <int WT, int kR, int kS, bool kOutF32, int kEpi>
-__global__ __launch_bounds__(kGemmMaxWaves * kWave) void gemm_kernel(
+__global__ __launch_bounds__(kGemmWaves * kWave) void gemm_kernel(
     const uint8_t* pk_W, const uint8_t* pk_x, const float* pk_w_scale, const void* pk_bias, int pk_M, int pk_K,
     int pk_B, int pk_col_tiles, int pk_steps, GemvArgs a) {
     using F = WFmt<WT>;
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(kGemmMaxWaves * kWave) void gemm_kernel(
     constexpr int RT = kR / 16;             // operands of rows
     constexpr int kPitch = kR + 4;          // floats; keeps 16-byte stores aligned and spreads the banks
     constexpr int kXP = F::kXBytes / 16;    // 16-byte pieces of x per weight chunk
-    constexpr int kIts = kR * kCols / (kGemmMinWaves * kWave);
+    constexpr int kIts = (kR * kCols + kGemmWaves * kWave - 1) / (kGemmWaves * kWave);
     static_assert(kR % 16 == 0, "whole operands");
     extern __shared__ float red[];          // [waves][kCols][kPitch]
     a.B = pk_B;
@@ -128,7 +130,6 @@ __global__ __launch_bounds__(kGemmMaxWaves * kWave) void gemm_kernel(
     const int K = pk_K;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int waves = blockDim.x / kWave;
     // The column tiles of a row tile sit next to each other on one XCD (workgroups x and x + 8),
     // so that its L2 fetches the row tile's weights once.
     const int j8 = blockIdx.x >> 3;
@@ -163,7 +164,8 @@ __global__ __launch_bounds__(kGemmMaxWaves * kWave) void gemm_kernel(
     // What the epilogue needs, requested behind the first block: this thread's row is the same in
     // every round of its store loop.
     const int mm = threadIdx.x % kR, m = m0 + mm;
-    const int bb0 = threadIdx.x / kR, bb_step = blockDim.x / kR;
+    const int bb0 = threadIdx.x / kR;
+    constexpr int bb_step = kGemmWaves * kWave / kR;
     const int mr = min(m, a.M - 1);
     const float braw = load_act<WT>(pk_bias ? pk_bias : (const void*)pk_x, pk_bias ? mr : 0);
     const float bias = pk_bias ? braw : 0.0f;
@@ -216,10 +218,9 @@ __global__ __launch_bounds__(kGemmMaxWaves * kWave) void gemm_kernel(
     for (int it = 0; it < kIts; ++it) {
         const int bb = bb0 + it * bb_step, b = b0 + bb;
         if (bb >= kCols || m >= a.M || b >= a.B) continue;
-        float p[kGemmMaxWaves];
+        float p[kGemmWaves];
 #pragma unroll
-        for (int w = 0; w < kGemmMaxWaves; ++w)
-            p[w] = w < kGemmMinWaves || w < waves ? red[(w * kCols + bb) * kPitch + mm] : 0.0f;
+        for (int w = 0; w < kGemmWaves; ++w) p[w] = red[(w * kCols + bb) * kPitch + mm];
         float pre = tree_sum(p) * ws + bias;
         const size_t o = (size_t)b * a.M + m;
         if (a.pre_gelu) store_res<kOutF32>(a.pre_gelu, o, pre);
@@ -518,7 +519,7 @@ bool gemm_takes(int w_dtype, int B, int M, int K) {
     if (B < from || K > (1 << 20)) return false;
     // Grids beyond 2^31 threads stay with gemv.hip.
     const long long groups = 8ll * ((M + 127) / 128) * ((B + 15) / 16);
-    return groups * kGemmMaxWaves * kWave < (1ll << 31);
+    return groups * kGemmWaves * kWave < (1ll << 31);
 }
 
 // The launch for arguments that launch_gemv has checked.  The waves split a row's steps alike
@@ -551,7 +552,7 @@ int launch_gemm(GemvArgs a, int w_dtype, bool out_f32, int epi, void* stream) {
             }
         }
     } else {
-        waves = steps <= kGemmSteps * kGemmMinWaves ? kGemmMinWaves : kGemmMaxWaves;
+        waves = kGemmWaves;
         last = (steps / waves) << 8 | (steps % waves);
         lds = (size_t)waves * p.cols * (p.rows + 4) * sizeof(float);
     }
