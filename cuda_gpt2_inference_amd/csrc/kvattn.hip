@@ -2331,6 +2331,8 @@ constexpr int kRagged8MidRows = 4096;
 struct Plan {
     int strategy, slots, seg_rows;
     bool lat;   // the latency shape: tiles of KVATTN_SPLIT_LAT_ROWS rows (else the streaming shape's)
+    int ws_slots;   // > 0: AUTO took fused_single for a split plan of so many slots (fused_many); the
+                    // workspace is checked as that plan's, though fused_single does not use it
 };
 
 // A call is latency bound while it streams fewer rows than kStreamRows (with per-sequence
@@ -2352,7 +2354,11 @@ bool latency_bound(int B, int NH, int total_rows, bool ragged = false, bool k8 =
 // only its first two cases).
 // - One segment per (b,h) (last-block instance, which then stores without a merge) when the
 //   heads alone give 192 or more workgroups and no head is longer than 512 rows; 8-bit caches
-//   take the streaming shape's 64-row tiles there.
+//   take the streaming shape's 64-row tiles there below 384 heads (INT8, 300 positions, us per
+//   call: 240 heads 6.52, 6.76 with the latency shape's; 576 heads 10.13, 9.24).  A contiguous
+//   INT8 cache also up to 1024 rows from kManyHeads heads on (700 positions, 480 heads: 12.1, 15.8
+//   in segments; 1024 positions, 768 heads: 19.7, 21.6); the other types take fused_single
+//   there (fused_many).
 // - The designated merger while its grid stays within kAutoDesignatedMaxGrid workgroups and
 //   the call streams at most kAutoDesignatedMaxBytes: segments of max(128, maxT / 16) rows
 //   (a power of two, so at most 16 per head; up to 64 per head when fewer than 12 heads
@@ -2374,10 +2380,11 @@ bool latency_bound(int B, int NH, int total_rows, bool ragged = false, bool k8 =
 //   packs two segments per workgroup on the general plan: 64 sequences of up to 8192
 //   positions ran 9 % slower on 256-row segments), keep the general plan (false).
 // Returns false to leave the plan to the general rules below.
+constexpr long long kManyHeads = 480;
 constexpr long long kAutoDesignatedMaxGrid = 768;
 constexpr long long kAutoDesignatedMaxBytes = 64ll << 20;
 constexpr long long kAutoDoubledMaxBytes = 40ll << 20;
-bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragged, Plan& p) {
+bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragged, bool paged, Plan& p) {
     const long long heads = (long long)B * NH;
     const bool k8 = is_8bit(kv_dtype);
     const long long row_bytes = kv_dtype == KVATTN_KV_F32 ? 512 : (kv_dtype == KVATTN_KV_BF16 ? 256 : 136);
@@ -2386,7 +2393,14 @@ bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragg
         p.strategy = KVATTN_SPLIT_LASTBLOCK;
         p.seg_rows = 512;
         p.slots = 1;
-        p.lat = !k8;
+        p.lat = !k8 || (!paged && heads >= 384);
+        return true;
+    }
+    if (!paged && kv_dtype == KVATTN_KV_INT8 && maxT <= 1024 && heads >= kManyHeads) {
+        p.strategy = KVATTN_SPLIT_LASTBLOCK;
+        p.seg_rows = 1024;
+        p.slots = 1;
+        p.lat = true;
         return true;
     }
     // At most 16 segments per head once the heads give 192 workgroups with them; fewer heads
@@ -2424,6 +2438,28 @@ bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragg
     return false;
 }
 
+// Many heads of up to 1024 positions fill the GPU by themselves: a workgroup a head, scores in LDS
+// (fused_single), saves the segments' partials and merge, and the second pass over the scores
+// costs less than an online softmax's rescaling.  us per call, a plan of segments / fused_single
+// (NH = 12, the plan made for the longest length; sequences x positions, u: all of that length,
+// r: U[1, that]):
+//   BF16  20 x 300 r 6.94 / 6.36, u 7.49 / 7.60   32 x 300 r 8.17 / 8.01, u 8.70 / 8.67   48 x 300 u 11.3 / 10.4
+//         40 x 700 u 18.9 / 16.1   48 x 1024 u 28.2 / 28.2, r 19.6 / 18.1   64 x 1024 u 35.2 / 32.4, r 23.2 / 21.0
+//         32 x 1024 r 13.18 / 13.19
+//   FP8   20 x 300 r 6.47 / 5.50   64 x 600 u 19.1 / 13.4   64 x 1024 u 21.1 / 18.4, r 16.6 / 13.9
+//         32 x 1024 r  9.89 / 11.48
+//   FP32  40 x 700 u 33.9 / 28.6   48 x 1024 r 30.2 / 31.9   64 x 1024 u 67.0 / 63.3   48 x 300 u 17.7 / 21.0
+//   INT8  48 x 1024 r 14.9 / 20.7 (its per-byte converts, done twice for no rescaling saved)
+bool fused_many(long long heads, int maxT, int total, int kv_dtype) {
+    if (total > 1024 || maxT > 2048) return false;
+    switch (kv_dtype) {
+        case KVATTN_KV_BF16: return heads >= (total <= 512 ? 384 : kManyHeads);
+        case KVATTN_KV_FP8_E4M3: return heads >= (total <= 512 ? 240 : kManyHeads);
+        case KVATTN_KV_F32: return total > 512 && heads >= (total <= 768 ? kManyHeads : 640);
+        default: return false;
+    }
+}
+
 // paged: a paged cache, which has no fused_single or cooperative instance and whose
 // segments start at multiples of 64 rows (the tile), so rows per segment are planned on
 // the device unless S < 0 gives a multiple of 64.
@@ -2439,6 +2475,15 @@ int make_plan(int B, int NH, int maxT, int len_hint, int S, int strategy, int kv
     }
     const int total_hint = (len_hint < 0 ? maxT - 1 : len_hint) + 1;
     const bool auto_strategy = strategy == KVATTN_AUTO;
+    if (auto_strategy && tuned && !paged && S == 0 && total_hint > kFusedMaxRows &&
+        fused_many((long long)B * NH, maxT, total_hint, kv_dtype)) {
+        KV_TRY(make_plan(B, NH, maxT, len_hint, S, strategy, kv_dtype, p, paged, ragged, false));
+        p.ws_slots = p.slots;
+        p.strategy = KVATTN_FUSED_SINGLE;
+        p.slots = 1;
+        p.seg_rows = 0;
+        return KVATTN_OK;
+    }
     if (strategy == KVATTN_AUTO) {
         // Short contexts: one workgroup per (b,h).  Otherwise split; a single launch with
         // the in-kernel merge while the whole call is latency bound, and split + merge
@@ -2457,7 +2502,7 @@ int make_plan(int B, int NH, int maxT, int len_hint, int S, int strategy, int kv
             // hinted lengths too, and segments longer than a paged wave walks).
             if (hinted || heads > 16 || heads * designated_slots(maxT, B * NH) > kDesignatedMaxGrid) {
                 Plan q{};
-                if (tuned_auto(B, NH, maxT, hinted ? total_hint : maxT, kv_dtype, ragged, q) &&
+                if (tuned_auto(B, NH, maxT, hinted ? total_hint : maxT, kv_dtype, ragged, paged, q) &&
                     (q.strategy != KVATTN_SPLIT_MERGE || (hinted && !paged)) &&
                     !(paged && q.seg_rows > kMaxPagedSegRows)) {
                     p = q;
@@ -2511,6 +2556,9 @@ int make_plan(int B, int NH, int maxT, int len_hint, int S, int strategy, int kv
 // append == true: the launch also writes the current token's K/V row (kvattn_append_decode).
 // pm != nullptr: kv / kv_scale are page pools addressed through pm's block table.
 // use_scratch: the workspace is the library's static device array (kvattn_decode_static).
+constexpr size_t kScratchBytes = 8u << 20;
+constexpr int kScratchMaxHeads = 16384;
+constexpr size_t kScratchCounterBytes = kScratchMaxHeads * sizeof(unsigned);
 int scratch_base(hipStream_t stream, uint8_t*& base);
 bool carve_scratch(uint8_t* base, int B, int NH, int S, Workspace& w);
 
@@ -2526,6 +2574,19 @@ int decode_impl(void* out, const void* qkv, const void* kv, const float* kv_scal
     hipStream_t stream = (hipStream_t)stream_v;
 
     if (plan.strategy == KVATTN_FUSED_SINGLE) {
+        if (plan.ws_slots > 0) {
+            const long long heads = (long long)B * NH;
+            if (use_scratch) {
+                if (heads > kScratchMaxHeads ||
+                    kvattn_layout::ws_layout(heads, plan.ws_slots, kScratchBytes, kScratchCounterBytes).bytes > kScratchBytes)
+                    return KVATTN_ERR_WORKSPACE;
+            } else {
+                if (!workspace) return KVATTN_ERR_WORKSPACE;
+                if (!aligned16(workspace)) return KVATTN_ERR_MISALIGNED;
+                if (kvattn_layout::ws_layout(heads, plan.ws_slots, workspace_bytes).bytes > workspace_bytes)
+                    return KVATTN_ERR_WORKSPACE;
+            }
+        }
         KV_TRY(resolve_len(d_cur_len));
         return launch_fused_single(out, qkv, kv, kv_scale, append ? const_cast<void*>(kv) : nullptr,
                                    append ? const_cast<float*>(kv_scale) : nullptr, B, NH, maxT, d_cur_len,
@@ -2626,9 +2687,6 @@ int decode_impl(void* out, const void* qkv, const void* kv, const float* kv_scal
 // (b,h) (so that calls of different B*NH never find another plan's partials where their
 // counters sit; the last-block kernels leave the counters at zero after every call), then
 // the partials and tagged words of the current plan (carved as in a caller's workspace).
-constexpr size_t kScratchBytes = 8u << 20;
-constexpr int kScratchMaxHeads = 16384;
-constexpr size_t kScratchCounterBytes = kScratchMaxHeads * sizeof(unsigned);
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
 // Device address of this device's `scratch`, found once per device with hipGetSymbolAddress

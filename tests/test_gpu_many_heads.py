@@ -1,0 +1,78 @@
+"""AUTO's plans for many heads of up to 1024 positions: fused_single (BF16, FP8, FP32) or one segment
+per head (INT8), against the split + merge strategy on the same inputs: uniform and ragged
+lengths, with and without a hint, appending, on either side of the rule's edges; and the workspace
+asked for as before."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+HS = 64
+
+
+@pytest.mark.parametrize("dtype,tol", [("f32", 1e-5), ("bf16", 1e-2), ("int8", 1e-2), ("fp8", 1e-2)])
+@pytest.mark.parametrize("B,NH,maxT", [(40, 12, 513), (60, 8, 1024), (60, 8, 1025), (479, 1, 700), (80, 6, 700),
+                                       (64, 10, 769), (48, 8, 300), (24, 10, 512)])
+@pytest.mark.parametrize("ragged,hint,append", [(False, True, False), (True, False, True), (True, True, False),
+                                                (False, False, True)])
+def test_many_heads_against_split_merge(dev, dtype, tol, B, NH, maxT, ragged, hint, append):
+    import torch
+    from cuda_gpt2_inference_amd import kvattn
+    g = torch.Generator(device=dev)
+    g.manual_seed(B * maxT)
+    act = torch.float32 if dtype == "f32" else torch.bfloat16
+    w8 = dtype in ("int8", "fp8")
+    shape = (2, B, NH, maxT, HS)
+    if w8:
+        cache = torch.randint(0, 120, shape, generator=g, device=dev, dtype=torch.uint8)
+        scale = 0.02 * torch.rand(shape[:-1], generator=g, device=dev)
+    else:
+        cache, scale = torch.randn(shape, generator=g, device=dev).to(act), None
+    qkv = torch.randn(B, 3, NH, HS, generator=g, device=dev).to(act)
+    if ragged:
+        cur = torch.randint(0, maxT, (B,), generator=g, device=dev, dtype=torch.int32)
+        cur[0], cur[1] = maxT - 1, 0
+    else:
+        cur = torch.tensor([maxT - 2], dtype=torch.int32, device=dev)
+    # Rows past the length are never cleared: NaNs there must not reach the output.
+    total = (cur.long() + 1) if ragged else (cur.long() + 1).expand(B)
+    dead = torch.arange(maxT, device=dev)[None] >= total[:, None]
+    if not w8:
+        cache.masked_fill_(dead[None, :, None, :, None], float("nan"))
+    else:
+        scale.masked_fill_(dead[None, :, None, :], float("nan"))
+    ws = kvattn.Workspace(B, NH, maxT)
+    kw = dict(kv_dtype=dtype, cur_len=cur, lens_per_seq=ragged, len_hint=maxT - (1 if ragged else 2) if hint else -1,
+              **ws.kwargs())
+    got = []
+    for strategy in ("auto", "split_merge"):
+        c, s = cache.clone(), None if scale is None else scale.clone()
+        out = torch.full((B, NH, HS), float("nan"), dtype=act, device=dev)
+        (kvattn.append_decode if append else kvattn.decode)(out, qkv, c, B, NH, HS, maxT, kv_scale=s, strategy=strategy,
+                                                            **kw)
+        torch.cuda.synchronize()
+        got.append((out.double().cpu().numpy(), c.view(torch.uint8).cpu(), None if s is None else s.view(torch.int32).cpu()))
+    a, b = got[0][0], got[1][0]
+    assert np.isfinite(a).all()
+    assert np.abs(a - b).max() <= tol * np.abs(b).max()
+    assert torch.equal(got[0][1], got[1][1])
+    if w8:
+        assert torch.equal(got[0][2], got[1][2])
+
+
+def test_many_heads_still_ask_for_a_workspace(dev):
+    import torch
+    from cuda_gpt2_inference_amd import kvattn
+    B, NH, maxT = 48, 12, 700
+    assert kvattn.plan(B, NH, HS, maxT, kv_dtype="bf16")[0] == kvattn.FUSED_SINGLE
+    cache = torch.zeros(2, B, NH, maxT, HS, dtype=torch.bfloat16, device=dev)
+    qkv = torch.zeros(B, 3, NH, HS, dtype=torch.bfloat16, device=dev)
+    out = torch.empty(B, NH, HS, dtype=torch.bfloat16, device=dev)
+    buf = torch.zeros(1 << 16, dtype=torch.uint8, device=dev)
+    for kw in ({}, dict(workspace=buf, workspace_nbytes=buf.numel())):
+        with pytest.raises(kvattn.KvAttnError) as e:
+            kvattn.decode(out, qkv, cache, B, NH, HS, maxT, kv_dtype="bf16", **kw)
+        assert e.value.status == kvattn.ERR_WORKSPACE
+    with pytest.raises(kvattn.KvAttnError) as e:
+        kvattn.decode(out, qkv, cache, B, NH, HS, maxT, kv_dtype="bf16", workspace=buf.data_ptr() + 4,
+                      workspace_nbytes=1 << 30)
+    assert e.value.status == kvattn.ERR_MISALIGNED
