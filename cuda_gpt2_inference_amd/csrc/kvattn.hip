@@ -2354,8 +2354,9 @@ bool latency_bound(int B, int NH, int total_rows, bool ragged = false, bool k8 =
 // only its first two cases).
 // - One segment per (b,h) (last-block instance, which then stores without a merge) when the
 //   heads alone give 192 or more workgroups and no head is longer than 512 rows; 8-bit caches
-//   take the streaming shape's 64-row tiles there below 384 heads (INT8, 300 positions, us per
-//   call: 240 heads 6.52, 6.76 with the latency shape's; 576 heads 10.13, 9.24).  A contiguous
+//   take the streaming shape's 64-row tiles there below 384 heads and from 1024 on (INT8, us per
+//   call, streaming / latency shape: 240 heads of 300 positions 6.52 / 6.76, 576 of 300 10.13 /
+//   9.24, 1536 of 400 18.2 / 19.4, 1152 of 1024 30.0 / 32.4).  A contiguous
 //   INT8 cache also up to 1024 rows from kManyHeads heads on (700 positions, 480 heads: 12.1, 15.8
 //   in segments; 1024 positions, 768 heads: 19.7, 21.6); the other types take fused_single
 //   there (fused_many).
@@ -2393,14 +2394,14 @@ bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragg
         p.strategy = KVATTN_SPLIT_LASTBLOCK;
         p.seg_rows = 512;
         p.slots = 1;
-        p.lat = !k8 || (!paged && heads >= 384);
+        p.lat = !k8 || (!paged && heads >= 384 && heads < 1024);
         return true;
     }
     if (!paged && kv_dtype == KVATTN_KV_INT8 && maxT <= 1024 && heads >= kManyHeads) {
         p.strategy = KVATTN_SPLIT_LASTBLOCK;
         p.seg_rows = 1024;
         p.slots = 1;
-        p.lat = true;
+        p.lat = heads < 1024;
         return true;
     }
     // At most 16 segments per head once the heads give 192 workgroups with them; fewer heads
