@@ -381,17 +381,21 @@ __global__ __launch_bounds__(kTallWaves * kWave) void gemm_tall_kernel(
     __syncthreads();
     if (!busy) return;
 
-    // FP32 sums: a block's four steps as a tree, blocks in turn to two sums.
-    F32x4 acc[2][NT];
+    // FP32 sums: a block's four steps as a tree; blocks in turn to two sums, or to one with 8-bit
+    // weights, which have half as many blocks (and no registers left for two with 64 tokens).
+    constexpr int kSets = F::k8bit ? 1 : 2;
+    F32x4 acc[kSets][NT];
     // Four outputs of a token in one store, where they are aligned.
     const bool vec_ok = (((uintptr_t)a.out | (uintptr_t)a.pre_gelu) & (kOutF32 ? 15u : 7u)) == 0;
     auto clear = [&]() {
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[0][j] = acc[1][j] = F32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int k = 0; k < kSets; ++k) acc[k][j] = F32x4{0.0f, 0.0f, 0.0f, 0.0f};
     };
     clear();
     auto consume = [&](Block& t, auto which) {
-        constexpr int q = decltype(which)::value;
+        constexpr int q = decltype(which)::value % kSets;
         const int st0 = blk * kT;
 #pragma unroll
         for (int u = 0; u < kT; u += 2) unpair(t.w[u], t.w[u + 1]);
@@ -423,7 +427,8 @@ __global__ __launch_bounds__(kTallWaves * kWave) void gemm_tall_kernel(
         const bool whole = M % 4 == 0 && m < M && vec_ok;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            const F32x4 sum = acc[0][j] + acc[1][j];
+            F32x4 sum = acc[0][j];
+            if constexpr (kSets == 2) sum += acc[1][j];
             const F32x4 v = __builtin_bit_cast(F32x4, from_lane(__builtin_bit_cast(U32x4, sum), back));
             const int b = b0 + 16 * j + lr;
             if (b >= B) continue;
