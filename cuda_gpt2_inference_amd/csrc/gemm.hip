@@ -382,8 +382,8 @@ __global__ __launch_bounds__(kTallWaves * kWave) void gemm_tall_kernel(
     if (!busy) return;
 
     // FP32 sums: a block's four steps as a tree; blocks in turn to two sums, or to one with 8-bit
-    // weights, which have half as many blocks (and no registers left for two with 64 tokens).
-    constexpr int kSets = F::k8bit ? 1 : 2;
+    // weights and 64 tokens, which leave no registers for two and have half as many blocks.
+    constexpr int kSets = F::k8bit && NT == 4 ? 1 : 2;
     F32x4 acc[kSets][NT];
     // Four outputs of a token in one store, where they are aligned.
     const bool vec_ok = (((uintptr_t)a.out | (uintptr_t)a.pre_gelu) & (kOutF32 ? 15u : 7u)) == 0;

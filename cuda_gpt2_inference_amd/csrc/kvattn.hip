@@ -2331,8 +2331,8 @@ constexpr int kRagged8MidRows = 4096;
 struct Plan {
     int strategy, slots, seg_rows;
     bool lat;   // the latency shape: tiles of KVATTN_SPLIT_LAT_ROWS rows (else the streaming shape's)
-    int ws_slots;   // > 0: AUTO took fused_single for a split plan of so many slots (fused_many); the
-                    // workspace is checked as that plan's, though fused_single does not use it
+    int ws_slots;   // > 0: AUTO took a plan for many heads (many_heads) in place of one of so many slots;
+                    // the workspace is checked as that plan's, though less of it, or none, is used
 };
 
 // A call is latency bound while it streams fewer rows than kStreamRows (with per-sequence
@@ -2356,10 +2356,7 @@ bool latency_bound(int B, int NH, int total_rows, bool ragged = false, bool k8 =
 //   heads alone give 192 or more workgroups and no head is longer than 512 rows; 8-bit caches
 //   take the streaming shape's 64-row tiles there below 384 heads and from 1024 on (INT8, us per
 //   call, streaming / latency shape: 240 heads of 300 positions 6.52 / 6.76, 576 of 300 10.13 /
-//   9.24, 1536 of 400 18.2 / 19.4, 1152 of 1024 30.0 / 32.4).  A contiguous
-//   INT8 cache also up to 1024 rows from kManyHeads heads on (700 positions, 480 heads: 12.1, 15.8
-//   in segments; 1024 positions, 768 heads: 19.7, 21.6); the other types take fused_single
-//   there (fused_many).
+//   9.24, 1536 of 400 18.2 / 19.4, 1152 of 1024 30.0 / 32.4).
 // - The designated merger while its grid stays within kAutoDesignatedMaxGrid workgroups and
 //   the call streams at most kAutoDesignatedMaxBytes: segments of max(128, maxT / 16) rows
 //   (a power of two, so at most 16 per head; up to 64 per head when fewer than 12 heads
@@ -2395,13 +2392,6 @@ bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragg
         p.seg_rows = 512;
         p.slots = 1;
         p.lat = !k8 || (!paged && heads >= 384 && heads < 1024);
-        return true;
-    }
-    if (!paged && kv_dtype == KVATTN_KV_INT8 && maxT <= 1024 && heads >= kManyHeads) {
-        p.strategy = KVATTN_SPLIT_LASTBLOCK;
-        p.seg_rows = 1024;
-        p.slots = 1;
-        p.lat = heads < 1024;
         return true;
     }
     // At most 16 segments per head once the heads give 192 workgroups with them; fewer heads
@@ -2450,24 +2440,46 @@ bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragg
 //   FP8   20 x 300 r 6.47 / 5.50   64 x 600 u 19.1 / 13.4   64 x 1024 u 21.1 / 18.4, r 16.6 / 13.9
 //         32 x 1024 r  9.89 / 11.48
 //   FP32  40 x 700 u 33.9 / 28.6   48 x 1024 r 30.2 / 31.9   64 x 1024 u 67.0 / 63.3   48 x 300 u 17.7 / 21.0
-//   INT8  48 x 1024 r 14.9 / 20.7 (its per-byte converts, done twice for no rescaling saved)
-bool fused_many(long long heads, int maxT, int total, int kv_dtype) {
-    if (total > 1024 || maxT > 2048) return false;
+//   INT8  48 x 1024 r 14.9 / 20.7 (twice the instructions per byte): one segment per head instead
+//         (last-block instance), 14.2; 40 x 700 u 15.8 / 12.1 in one segment; 64 x 1024 u 21.6 / 19.7
+// Returns whether the plan p, made without this rule, is replaced.
+// known: the host knows the longest length, or every sequence has its own.  (One unknown length for
+// all of up to 769-1024 BF16 positions keeps its device-planned segments: 576 heads u 28.2 / 28.2,
+// 1152 50.9 / 48.9.)
+// FP8 up to 512 positions and FP32 beyond 768 differ with ragged (every sequence its own length): 128 x 400
+// FP8 u 17.3 / 17.8, r 15.2 / 14.1; FP32 56 x 1024 u 60.6 / 57.3, 64 x 1024 r 42.9 / 44.5, 96 x 1024 r 53.2 / 51.8.
+bool many_heads(long long heads, int maxT, int total, int kv_dtype, bool known, bool ragged, Plan& p) {
+    bool fused = total <= 1024 && maxT <= 2048;
     switch (kv_dtype) {
-        case KVATTN_KV_BF16: return heads >= (total <= 512 ? 384 : kManyHeads);
-        case KVATTN_KV_FP8_E4M3: return heads >= (total <= 512 ? 240 : kManyHeads);
-        case KVATTN_KV_F32: return total > 512 && heads >= (total <= 768 ? kManyHeads : 640);
-        default: return false;
+        case KVATTN_KV_BF16:
+            fused = fused && heads >= (total <= 512 ? 384 : kManyHeads) && (known || total <= 768);
+            break;
+        case KVATTN_KV_FP8_E4M3:
+            fused = fused && (total > 512 ? heads >= kManyHeads : heads >= 240 && (ragged || heads < 1024));
+            break;
+        case KVATTN_KV_F32:
+            fused = fused && total > 512 && heads >= (total <= 768 ? kManyHeads : ragged ? 1024 : 640);
+            break;
+        default: fused = false; break;
     }
+    if (fused) {
+        p = Plan{KVATTN_FUSED_SINGLE, 1, 0, p.lat, p.slots};
+        return true;
+    }
+    if (kv_dtype == KVATTN_KV_INT8 && maxT > 512 && maxT <= 1024 && heads >= kManyHeads) {
+        p = Plan{KVATTN_SPLIT_LASTBLOCK, 1, 1024, heads < 1024, p.slots};
+        return true;
+    }
+    return false;
 }
 
 // paged: a paged cache, which has no fused_single or cooperative instance and whose
 // segments start at multiples of 64 rows (the tile), so rows per segment are planned on
 // the device unless S < 0 gives a multiple of 64.
 // ragged: per-sequence lengths.  tuned: AUTO may take tuned_auto's plan (off: the general
-// rules alone).
+// rules alone).  many: and many_heads may replace it.
 int make_plan(int B, int NH, int maxT, int len_hint, int S, int strategy, int kv_dtype, Plan& p,
-              bool paged = false, bool ragged = false, bool tuned = true) {
+              bool paged = false, bool ragged = false, bool tuned = true, bool many = true) {
     if (strategy < KVATTN_AUTO || strategy > KVATTN_SPLIT_DESIGNATED) return KVATTN_ERR_STRATEGY;
     if (len_hint >= maxT || len_hint < -1) return KVATTN_ERR_LENGTH;
     if (paged) {
@@ -2476,13 +2488,9 @@ int make_plan(int B, int NH, int maxT, int len_hint, int S, int strategy, int kv
     }
     const int total_hint = (len_hint < 0 ? maxT - 1 : len_hint) + 1;
     const bool auto_strategy = strategy == KVATTN_AUTO;
-    if (auto_strategy && tuned && !paged && S == 0 && total_hint > kFusedMaxRows &&
-        fused_many((long long)B * NH, maxT, total_hint, kv_dtype)) {
-        KV_TRY(make_plan(B, NH, maxT, len_hint, S, strategy, kv_dtype, p, paged, ragged, false));
-        p.ws_slots = p.slots;
-        p.strategy = KVATTN_FUSED_SINGLE;
-        p.slots = 1;
-        p.seg_rows = 0;
+    if (auto_strategy && tuned && many && !paged && S == 0 && total_hint > kFusedMaxRows) {
+        KV_TRY(make_plan(B, NH, maxT, len_hint, S, strategy, kv_dtype, p, paged, ragged, true, false));
+        many_heads((long long)B * NH, maxT, total_hint, kv_dtype, ragged || len_hint >= 0, ragged, p);
         return KVATTN_OK;
     }
     if (strategy == KVATTN_AUTO) {
@@ -2574,20 +2582,23 @@ int decode_impl(void* out, const void* qkv, const void* kv, const float* kv_scal
     KV_TRY(make_plan(B, NH, maxT, len_hint, S, strategy, kv_dtype, plan, pm != nullptr, lens_per_seq != 0));
     hipStream_t stream = (hipStream_t)stream_v;
 
-    if (plan.strategy == KVATTN_FUSED_SINGLE) {
-        if (plan.ws_slots > 0) {
-            const long long heads = (long long)B * NH;
-            if (use_scratch) {
-                if (heads > kScratchMaxHeads ||
-                    kvattn_layout::ws_layout(heads, plan.ws_slots, kScratchBytes, kScratchCounterBytes).bytes > kScratchBytes)
-                    return KVATTN_ERR_WORKSPACE;
-            } else {
-                if (!workspace) return KVATTN_ERR_WORKSPACE;
-                if (!aligned16(workspace)) return KVATTN_ERR_MISALIGNED;
-                if (kvattn_layout::ws_layout(heads, plan.ws_slots, workspace_bytes).bytes > workspace_bytes)
-                    return KVATTN_ERR_WORKSPACE;
-            }
+    if (plan.ws_slots > 0) {
+        const long long heads = (long long)B * NH;
+        if (use_scratch) {
+            auto fits = [&](int slots) {
+                return kvattn_layout::ws_layout(heads, slots, kScratchBytes, kScratchCounterBytes).bytes <= kScratchBytes;
+            };
+            Plan general{};
+            KV_TRY(make_plan(B, NH, maxT, len_hint, S, strategy, kv_dtype, general, false, lens_per_seq != 0, false));
+            if (heads > kScratchMaxHeads || !(fits(plan.ws_slots) || fits(general.slots))) return KVATTN_ERR_WORKSPACE;
+        } else {
+            if (!workspace) return KVATTN_ERR_WORKSPACE;
+            if (!aligned16(workspace)) return KVATTN_ERR_MISALIGNED;
+            if (kvattn_layout::ws_layout(heads, plan.ws_slots, workspace_bytes).bytes > workspace_bytes)
+                return KVATTN_ERR_WORKSPACE;
         }
+    }
+    if (plan.strategy == KVATTN_FUSED_SINGLE) {
         KV_TRY(resolve_len(d_cur_len));
         return launch_fused_single(out, qkv, kv, kv_scale, append ? const_cast<void*>(kv) : nullptr,
                                    append ? const_cast<float*>(kv_scale) : nullptr, B, NH, maxT, d_cur_len,

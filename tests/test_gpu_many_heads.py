@@ -11,7 +11,8 @@ HS = 64
 
 @pytest.mark.parametrize("dtype,tol", [("f32", 1e-5), ("bf16", 1e-2), ("int8", 1e-2), ("fp8", 1e-2)])
 @pytest.mark.parametrize("B,NH,maxT", [(40, 12, 513), (60, 8, 1024), (60, 8, 1025), (479, 1, 700), (80, 6, 700),
-                                       (64, 10, 769), (48, 8, 300), (24, 10, 512)])
+                                       (64, 10, 769), (48, 8, 300), (24, 10, 512), (128, 8, 300),
+                                       (86, 12, 800)])
 @pytest.mark.parametrize("ragged,hint,append", [(False, True, False), (True, False, True), (True, True, False),
                                                 (False, False, True)])
 def test_many_heads_against_split_merge(dev, dtype, tol, B, NH, maxT, ragged, hint, append):
@@ -76,3 +77,27 @@ def test_many_heads_still_ask_for_a_workspace(dev):
         kvattn.decode(out, qkv, cache, B, NH, HS, maxT, kv_dtype="bf16", workspace=buf.data_ptr() + 4,
                       workspace_nbytes=1 << 30)
     assert e.value.status == kvattn.ERR_MISALIGNED
+
+
+def test_many_heads_accept_the_replaced_plans_workspace(dev):
+    """A workspace of exactly what the replaced plan needs stays enough: one slot per head up to 512
+    positions (FP8), and the static array where that plan fitted."""
+    import torch
+    from cuda_gpt2_inference_amd import kvattn
+    B, NH, maxT = 24, 10, 512
+    assert kvattn.plan(B, NH, HS, maxT, kv_dtype="fp8", len_hint=299)[0] == kvattn.FUSED_SINGLE
+    cache = torch.zeros(2, B, NH, maxT, HS, dtype=torch.uint8, device=dev)
+    scale = torch.ones(2, B, NH, maxT, device=dev)
+    qkv = torch.ones(B, 3, NH, HS, dtype=torch.bfloat16, device=dev)
+    out = torch.empty(B, NH, HS, dtype=torch.bfloat16, device=dev)
+    cur = torch.tensor([299], dtype=torch.int32, device=dev)
+    n = kvattn.workspace_bytes(B, NH, HS, maxT, 1)
+    ws = torch.zeros(n, dtype=torch.uint8, device=dev)
+    kw = dict(kv_dtype="fp8", kv_scale=scale, cur_len=cur, len_hint=299)
+    kvattn.decode(out, qkv, cache, B, NH, HS, maxT, workspace=ws, workspace_nbytes=n, **kw)
+    kvattn.decode_static(out, qkv, cache, B, NH, HS, maxT, **kw)
+    torch.cuda.synchronize()
+    assert not out.any()
+    with pytest.raises(kvattn.KvAttnError) as e:
+        kvattn.decode(out, qkv, cache, B, NH, HS, maxT, workspace=ws, workspace_nbytes=n - 4096, **kw)
+    assert e.value.status == kvattn.ERR_WORKSPACE
