@@ -68,8 +68,10 @@ typedef enum kvattn_dtype {
 } kvattn_dtype;
 
 typedef enum kvattn_strategy {
-    KVATTN_AUTO = 0,                /* fused_single for short contexts, else a split plan
-                                       chosen from len_hint, the shape and the cache type:
+    KVATTN_AUTO = 0,                /* fused_single for short contexts and for many heads of
+                                       up to 1024 positions (contiguous F32, BF16 and FP8
+                                       caches), else a split plan chosen from len_hint, the
+                                       shape and the cache type:
                                        the designated merger while its grid is small, one
                                        segment per (b,h) for many short heads, split +
                                        merge kernels once the call is bandwidth bound */
