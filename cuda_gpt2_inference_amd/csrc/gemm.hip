@@ -509,18 +509,25 @@ GemmPlan gemm_plan(int B, int M, int K, bool out_f32, int epi) {
 
 namespace kvattn_internal {
 
-// Whether a call takes the matrix cores.  Measured against gemv.hip (us per call, graph of calls,
-// MI355X; rows x K, tokens):
-//   BF16  768 x 768    3: 3.7 / 3.0   16: 10.5 / 3.0   64: 35.9 / 3.2
-//         768 x 3072   2: 4.3 / 4.9    3:  5.2 / 5.1   64: 55.2 / 5.4
-//   INT8  768 x 3072   2: 3.9 / 4.3    3:  4.7 / 4.7   64: 50.1 / 5.0
-//   FP32  768 x 768    3: 3.8 / 4.3    4:  4.2 / 4.3   64: 34.1 / 4.6
-//         768 x 3072   6: 9.2 / 10.5   8: 11.0 / 10.5  64: 59.0 / 11.1
-//         1600 x 6400  3: 27.7 / 24.6 (gemv.hip takes rows this long in blocks)
-// So from 3 tokens on; FP32 weights, whose MFMA does a sixteenth of the work, from 4, and from 8
-// where a row is long but still one block of gemv.hip.
+// Whether a call takes the matrix cores.  Measured, gemv.hip / this file (us per call, graph of
+// calls, MI355X; rows x K, tokens):
+//   BF16  768 x 768    2: 2.8 / 2.9   3: 3.7 / 2.9   768 x 3072  4: 4.8 / 5.1   5: 5.3 / 5.1
+//   FP8   768 x 768    2: 2.5 / 2.7   768 x 3072  2: 3.4 / 4.3   4: 4.4 / 4.3
+//   INT8  768 x 3072   2: 3.2 / 4.6   3: 3.5 / 4.6
+//   FP32  768 x 768    5: 3.9 / 4.3   7: 4.7 / 4.3   768 x 3072  5: 6.4 / 10.5  7: 7.5 / 11.9
+//         1280 x 5120  4: 28.6 / 20.1 (gemv.hip takes rows this long in blocks)
+// So from 3 tokens on.  Few rows (at most 1024: 64 tiles here) of more than 1600 but still one block
+// of gemv.hip leave most of the chip idle here, and stay there for 2 (8-bit weights: 1) tokens
+// more.  FP32 weights, whose MFMA does a sixteenth of the work: 4; few rows up to 1024 long 6; 8
+// beyond 1600, few 12.
 bool gemm_takes(int w_dtype, int B, int M, int K) {
-    const int from = w_dtype != KVATTN_KV_F32 ? 3 : (K > 1600 && K <= 4096 ? 8 : 4);
+    const bool few = M <= 1024, mid = K > 1600 && K <= 4096;
+    int from = 3;
+    switch (w_dtype) {
+        case KVATTN_KV_F32: from = mid ? (few ? 12 : 8) : (few && K <= 1024 ? 6 : 4); break;
+        case KVATTN_KV_BF16: from = few && mid ? 5 : 3; break;
+        default: from = few && mid ? 4 : 3; break;
+    }
     if (B < from || K > (1 << 20)) return false;
     // Grids beyond 2^31 threads stay with gemv.hip.
     const long long groups = 8ll * ((M + 127) / 128) * ((B + 15) / 16);

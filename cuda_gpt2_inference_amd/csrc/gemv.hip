@@ -91,12 +91,16 @@ __device__ __forceinline__ size_t cache_row(const GemvArgs& a, int b, int part, 
 // epilogue takes the dispatch id and the queue pointer (its tag) in user SGPRs, which leaves 10
 // dwords of preloaded arguments: W, x, the scales, the bias, M and K, all its first loads
 // need; B and out follow.
-template <int WT, int kC, int kR, bool kOutF32, int kEpi>
+// kPre: several vectors over a row of one block; the next vector's x is requested before this
+// one's products, else each vector waits a round trip to L2 (768 x 3072, us: BF16 2 vectors 4.34,
+// 3.71 with; FP32 5 vectors 8.17, 6.37 with).
+template <int WT, int kC, int kR, bool kOutF32, int kEpi, bool kPre = false>
 __global__ __launch_bounds__(kGemvWaves * kWave) void gemv_kernel(const uint8_t* pk_W, const uint8_t* pk_x,
                                                                   const float* pk_w_scale, const void* pk_bias,
                                                                   int pk_M, int pk_K, int pk_B, void* pk_out,
                                                                   GemvArgs a) {
     static_assert(kR * kC <= kGemvMaxRowChunks && (kR == 1 || kR == 2 || kR == 4), "weight registers");
+    static_assert(!kPre || (kR == 1 && kEpi != kEpiAppend8), "vectors in turn");
     static_assert(kEpi == kEpiNone || kR == 1, "the QKV epilogue takes one row per wave");
     a.W = pk_W;
     a.x = pk_x;
@@ -165,11 +169,18 @@ __global__ __launch_bounds__(kGemvWaves * kWave) void gemv_kernel(const uint8_t*
     }
     const int len0 = kEpi != kEpiNone ? a.cur_len[0] : 0;   // the QKV epilogue's column
     for (int b = 0; b < a.B; ++b) {
+        XRaw<WT> xn[kPre ? kC : 1];
+        if (kPre && b + 1 < a.B) {
+            const uint8_t* xb = a.x + (size_t)(b + 1) * a.K * kActBytes;
+#pragma unroll
+            for (int i = 0; i < (kPre ? kC : 0); ++i)
+                xn[i] = load_x<WT>(xb + (size_t)min(lane + i * kWave, nch - 1) * F::kXBytes);
+        }
         float accr[kR];
 #pragma unroll
         for (int r = 0; r < kR; ++r) accr[r] = 0.0f;
-        for (int kb = 0; kb < nblk; ++kb) {
-            if (kb > 0 || b > 0) {
+        for (int kb = 0; kb < (kPre ? 1 : nblk); ++kb) {
+            if (!kPre && (kb > 0 || b > 0)) {
                 if (nblk > 1) load_w(kb);   // one block: the weights stay in registers for every vector
                 load_xs(b, kb);
             }
@@ -278,6 +289,10 @@ __global__ __launch_bounds__(kGemvWaves * kWave) void gemv_kernel(const uint8_t*
                 }
             }
         }
+        if (kPre && b + 1 < a.B) {
+#pragma unroll
+            for (int i = 0; i < (kPre ? kC : 0); ++i) xr[i] = xn[i];
+        }
     }
 }
 
@@ -291,8 +306,32 @@ __global__ __launch_bounds__(kGemvWaves * kWave) void gemv_kernel(const uint8_t*
 #endif
 constexpr int kGemvTallRows = KVATTN_GEMV_TALL_ROWS;
 
+// Most chunks per lane for which the next vector's x fits the registers beside this one's.
+template <int WT> constexpr int kPreMaxChunks = WT == KVATTN_KV_F32 ? 16 : WT == KVATTN_KV_BF16 ? 8 : 4;
+
+// One row per wave.  3, 6 and 12 chunks beside the powers of two: a lane's chunks beyond the row are
+// loaded and multiplied for nothing (768 x 3072, one vector, 8 / 6 chunks BF16 3.56 / 3.25 us, 4 / 3
+// FP8 3.11 / 2.95, 16 / 12 FP32 4.17 / 4.04).
+template <int WT, bool kOut, int kEpi, bool kPre>
+const void* gemv_row_ptr(int chunks_per_lane) {
+    constexpr int kMax = kPre ? kPreMaxChunks<WT> : kGemvMaxChunks;
+    if (chunks_per_lane <= 1) return (const void*)&gemv_kernel<WT, 1, 1, kOut, kEpi, kPre>;
+    if (chunks_per_lane <= 2) return (const void*)&gemv_kernel<WT, 2, 1, kOut, kEpi, kPre>;
+    if (chunks_per_lane <= 3) return (const void*)&gemv_kernel<WT, 3, 1, kOut, kEpi, kPre>;
+    if (kMax == 4 || chunks_per_lane <= 4) return (const void*)&gemv_kernel<WT, 4, 1, kOut, kEpi, kPre>;
+    if constexpr (kMax >= 8) {
+        if (chunks_per_lane <= 6) return (const void*)&gemv_kernel<WT, 6, 1, kOut, kEpi, kPre>;
+        if (kMax == 8 || chunks_per_lane <= 8) return (const void*)&gemv_kernel<WT, 8, 1, kOut, kEpi, kPre>;
+    }
+    if constexpr (kMax >= 16) {
+        if (chunks_per_lane <= 12) return (const void*)&gemv_kernel<WT, 12, 1, kOut, kEpi, kPre>;
+        return (const void*)&gemv_kernel<WT, 16, 1, kOut, kEpi, kPre>;
+    }
+    return nullptr;
+}
+
 template <int WT, bool kOut, int kEpi>
-const void* gemv_ptr(int chunks_per_lane, int rows) {
+const void* gemv_ptr(int chunks_per_lane, int rows, int vectors) {
     if constexpr (kEpi == kEpiNone) {
         if constexpr (WFmt<WT>::k8bit) {
             if (rows == 4) {
@@ -307,25 +346,24 @@ const void* gemv_ptr(int chunks_per_lane, int rows) {
             return (const void*)&gemv_kernel<WT, 8, 2, kOut, kEpi>;
         }
     }
-    if (chunks_per_lane <= 1) return (const void*)&gemv_kernel<WT, 1, 1, kOut, kEpi>;
-    if (chunks_per_lane <= 2) return (const void*)&gemv_kernel<WT, 2, 1, kOut, kEpi>;
-    if (chunks_per_lane <= 4) return (const void*)&gemv_kernel<WT, 4, 1, kOut, kEpi>;
-    if (chunks_per_lane <= 8) return (const void*)&gemv_kernel<WT, 8, 1, kOut, kEpi>;
-    return (const void*)&gemv_kernel<WT, kGemvMaxChunks, 1, kOut, kEpi>;
+    if constexpr (kEpi != kEpiAppend8)
+        if (vectors > 1 && chunks_per_lane <= kPreMaxChunks<WT>)
+            return gemv_row_ptr<WT, kOut, kEpi, true>(chunks_per_lane);
+    return gemv_row_ptr<WT, kOut, kEpi, false>(chunks_per_lane);
 }
 
 // The QKV epilogue writes qkv in the activation type, so only the plain GEMV takes another
 // output type.
 template <int WT>
-const void* gemv_ptr_out(int chunks_per_lane, int rows, bool out_f32, int epi) {
+const void* gemv_ptr_out(int chunks_per_lane, int rows, int vectors, bool out_f32, int epi) {
     constexpr bool kAct = WFmt<WT>::kActF32;
-    if (epi == kEpiAppend) return gemv_ptr<WT, kAct, kEpiAppend>(chunks_per_lane, 1);
+    if (epi == kEpiAppend) return gemv_ptr<WT, kAct, kEpiAppend>(chunks_per_lane, 1, vectors);
     if (epi == kEpiAppend8) {
         if constexpr (kAct) return nullptr;   // 8-bit caches sit behind bf16 activations
-        else return gemv_ptr<WT, false, kEpiAppend8>(chunks_per_lane, 1);
+        else return gemv_ptr<WT, false, kEpiAppend8>(chunks_per_lane, 1, vectors);
     }
-    return out_f32 ? gemv_ptr<WT, true, kEpiNone>(chunks_per_lane, rows)
-                   : gemv_ptr<WT, false, kEpiNone>(chunks_per_lane, rows);
+    return out_f32 ? gemv_ptr<WT, true, kEpiNone>(chunks_per_lane, rows, vectors)
+                   : gemv_ptr<WT, false, kEpiNone>(chunks_per_lane, rows, vectors);
 }
 
 }  // namespace
@@ -365,10 +403,10 @@ int launch_gemv(GemvArgs a, int w_dtype, bool out_f32, void* stream) {
     const int rows = a.kv || M < kGemvTallRows ? 1 : (w8 ? 4 : 2);
     const void* fn = nullptr;
     switch (w_dtype) {
-        case KVATTN_KV_F32: fn = gemv_ptr_out<KVATTN_KV_F32>(per_lane, rows, out_f32, epi); break;
-        case KVATTN_KV_BF16: fn = gemv_ptr_out<KVATTN_KV_BF16>(per_lane, rows, out_f32, epi); break;
-        case KVATTN_KV_INT8: fn = gemv_ptr_out<KVATTN_KV_INT8>(per_lane, rows, out_f32, epi); break;
-        default: fn = gemv_ptr_out<KVATTN_KV_FP8_E4M3>(per_lane, rows, out_f32, epi); break;
+        case KVATTN_KV_F32: fn = gemv_ptr_out<KVATTN_KV_F32>(per_lane, rows, B, out_f32, epi); break;
+        case KVATTN_KV_BF16: fn = gemv_ptr_out<KVATTN_KV_BF16>(per_lane, rows, B, out_f32, epi); break;
+        case KVATTN_KV_INT8: fn = gemv_ptr_out<KVATTN_KV_INT8>(per_lane, rows, B, out_f32, epi); break;
+        default: fn = gemv_ptr_out<KVATTN_KV_FP8_E4M3>(per_lane, rows, B, out_f32, epi); break;
     }
     if (!fn) return KVATTN_ERR_DTYPE;
     long long groups = ((M + rows - 1) / rows + kGemvWaves - 1) / kGemvWaves;

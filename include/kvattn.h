@@ -376,7 +376,7 @@ int kvattn_paged_decode(void* out, const void* qkv, void* pages, float* page_sca
  * Replaces launch_GEMV6_fused (Inference_gpt2/GEMV.cuh:132-206) and launch_GEMV6_w8x2
  * (Inference_gpt2/GEMV_w8.cuh:64-184), which matmul_forward[_w8] calls for one decode token
  * (inference_gpt2_opt.cu:106-132); the attention output projection is at :349-355.  Batches
- * (from 3 vectors on, FP32 weights from 4 or 8) go through the matrix cores with FP32 sums, where the reference takes cuBLASLt; other B > 1 read the weights once for all B
+ * (from 3 vectors on; few long rows 4 or 5, FP32 weights 4 to 12) go through the matrix cores with FP32 sums, where the reference takes cuBLASLt; other B > 1 read the weights once for all B
  * vectors when a row fits in one block.  A vector's result may differ in its last bits with
  * the size of the batch (another order of the same sums). */
 int kvattn_gemv(void* out, void* pre_gelu, const void* W, const float* w_scale, const void* x,

@@ -1,0 +1,63 @@
+"""The one-wave-per-row projection over a few vectors: each vector's result is the one it has alone,
+bit for bit (the same products in the same order), at the edges of the chunks a lane holds, with
+the last wave partly beyond the rows, GELU with the pre-activation, and the cache append."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "int8", "fp8"])
+@pytest.mark.parametrize("lane_chunks", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13, 16, 17])
+@pytest.mark.parametrize("edge", [-16, 0])
+def test_vectors_are_those_of_single_calls(dev, dtype, lane_chunks, edge):
+    import torch
+    from cuda_gpt2_inference_amd import kvattn
+    per = {"f32": 4, "bf16": 8}.get(dtype, 16)
+    K, M = 64 * per * lane_chunks + edge, 37
+    # Vectors that stay with this kernel: FP32 7 over rows of 1600 < K <= 4096, else 3.
+    B = 2 if dtype != "f32" else (7 if 1600 < K <= 4096 else 3)
+    g = torch.Generator(device=dev)
+    g.manual_seed(K)
+    act = torch.float32 if dtype == "f32" else torch.bfloat16
+    x = torch.randn(B, K, generator=g, device=dev).to(act)
+    bias = torch.randn(M, generator=g, device=dev).to(act)
+    scale = None
+    if dtype in ("int8", "fp8"):
+        W = torch.randint(0, 120, (M, K), generator=g, device=dev, dtype=torch.uint8)
+        scale = 1e-3 * torch.rand(M, generator=g, device=dev)
+    else:
+        W = torch.randn(M, K, generator=g, device=dev).to(act)
+    kw = dict(w_dtype=dtype, w_scale=scale, bias=bias, gelu=True)
+    got = [torch.full((B, M), float("nan"), dtype=act, device=dev) for _ in range(2)]
+    kvattn.gemv(got[0], W, x, B, M, K, pre_gelu=got[1], **kw)
+    for b in range(B):
+        one = [torch.full((1, M), float("nan"), dtype=act, device=dev) for _ in range(2)]
+        kvattn.gemv(one[0], W, x[b:b + 1].contiguous(), 1, M, K, pre_gelu=one[1], **kw)
+        torch.cuda.synchronize()
+        for o, w in zip(one, got):
+            assert torch.isfinite(o).all() and torch.equal(o[0], w[b])
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_append_of_two_vectors(dev, dtype):
+    import torch
+    from cuda_gpt2_inference_amd import kvattn
+    B, NH, maxT, K = 2, 12, 16, 768
+    g = torch.Generator(device=dev)
+    g.manual_seed(1)
+    act = torch.float32 if dtype == "f32" else torch.bfloat16
+    x = torch.randn(B, K, generator=g, device=dev).to(act)
+    W = torch.randn(3 * K, K, generator=g, device=dev).to(act)
+    cur = torch.tensor([3, 15], dtype=torch.int32, device=dev)
+    qkv = torch.empty(B, 3 * K, dtype=act, device=dev)
+    cache = torch.zeros(2, B, NH, maxT, 64, dtype=act, device=dev)
+    kvattn.gemv_qkv_append(qkv, W, x, B, NH, 64, K, cache, maxT, w_dtype=dtype, cur_len=cur,
+                           lens_per_seq=True)
+    ref = torch.empty_like(qkv)
+    kvattn.gemv(ref, W, x, B, 3 * K, K, w_dtype=dtype)
+    torch.cuda.synchronize()
+    assert torch.equal(qkv, ref)
+    want = torch.zeros_like(cache)
+    for b, t in enumerate((3, 15)):
+        want[:, b, :, t] = ref[b].view(3, NH, 64)[1:]
+    assert torch.equal(cache, want)
