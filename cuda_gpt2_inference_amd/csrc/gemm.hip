@@ -280,11 +280,16 @@ constexpr int kTallStage = 8;    // 16-byte token loads in flight per lane while
 constexpr int kTallWaves = 16;
 constexpr int kTallRows = 20000;           // from this many rows on (gemm_plan)
 constexpr int kTallGroups = 256;           // workgroups: one per CU
-constexpr long long kTallLds = 144 * 1024;
+// A row whose steps do not fill its last block gets one more step of zero tokens, which the block's
+// steps beyond the row multiply: with a real step's tokens there an infinity times their zero
+// weights would be NaN (and leaving those products out by a branch spills 23 to 79 registers).
+__host__ __device__ constexpr int tall_steps(int nsteps) { return nsteps + (nsteps % kTallSteps != 0 ? 1 : 0); }
+constexpr long long kTallLds = 144 * 1024;   // tokens, without that step
 // LDS of NT token tiles.
 template <int WT> constexpr long long tall_lds(int K, int NT) {
     return ((long long)K * WFmt<WT>::kWBytes / 16 + 3) / 4 * NT * kWave * WFmt<WT>::kXBytes;
 }
+constexpr int kTallLdsMax = 160 * 1024;      // with it: 144 KiB and a step of at most 8 KiB
 
 template <bool kOutF32>
 __device__ __forceinline__ void store_res4(void* p, size_t i, const float (&v)[4]) {
@@ -355,8 +360,8 @@ __global__ __launch_bounds__(kTallWaves * kWave) void gemm_tall_kernel(
         }
     };
     load_rows();
-    // Tokens to LDS: chunk c of token t of tile j goes to step c / 4, lane 16 (c % 4) + t.
-    const int pieces = nsteps * NT;
+    // Tokens to LDS: chunk c of token t of tile j goes to step c / 4, lane 16 (c % 4) + t; zeros beyond the row.
+    const int pieces = tall_steps(nsteps) * NT;
     for (int i0 = wave; i0 < pieces; i0 += kW * kPieces) {
         U32x4 v[kPieces][kXP];
 #pragma unroll
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(kTallWaves * kWave) void gemm_tall_kernel(
         F32x4 even[NT], pair[NT];
 #pragma unroll
         for (int u = 0; u < kT; ++u) {
-            const int st = min(st0 + u, nsteps - 1);   // steps beyond the row: zero weights
+            const int st = min(st0 + u, nsteps);   // beyond the row: the step of zeros
             const U32x4 wv = from_lane(t.w[u], src);
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
@@ -555,9 +560,9 @@ int launch_gemm(GemvArgs a, int w_dtype, bool out_f32, int epi, void* stream) {
     if (p.tall) {
         waves = kTallWaves;
         last = groups = std::min(groups, kTallGroups);
-        lds = (size_t)steps * (p.cols / 16) * kWave * (wbytes == 1 ? 32 : 16);
+        lds = (size_t)tall_steps(steps) * (p.cols / 16) * kWave * (wbytes == 1 ? 32 : 16);
         if (lds > 64 * 1024) {
-            const hipError_t e = hipFuncSetAttribute(p.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kTallLds);
+            const hipError_t e = hipFuncSetAttribute(p.fn, hipFuncAttributeMaxDynamicSharedMemorySize, kTallLdsMax);
             if (e != hipSuccess) {
                 set_last_hip_error((int)e);
                 return KVATTN_ERR_HIP;

@@ -126,6 +126,34 @@ def test_batch_special_values(dev, dtype):
             assert np.all(np.abs(one.astype(np.float64) - whole[b]) <= bound), b
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "int8", "fp8"])
+@pytest.mark.parametrize("B,M,K", [(16, 20000, 320), (20, 20001, 320), (40, 20000, 336), (20, 20000, 704),
+                                   (40, 20000, 960), (18, 65537, 80), (40, 20000, 1152), (20, 48, 336)])
+def test_special_values_in_the_last_steps_of_a_row(dev, dtype, B, M, K):
+    """Infinities and NaNs in a row's last step and last chunk, where the row's steps do not fill
+    the blocks of the kernel with tokens in LDS (M >= 20000; 48 rows: 16 x 16 tiles): each token as
+    that token alone (the vector units' path), and the other tokens within the bound.  The last
+    token keeps its own infinity behind a partial step's zeros."""
+    import torch
+    d, h = _make(dtype, B, M, K, seed=11, with_bias=False)
+    x = d["x"].reshape(B, K).clone()
+    x[1, K - 1], x[2, K - 20], x[3, K - 5], x[4, 0] = float("inf"), float("-inf"), float("nan"), float("inf")
+    x[B - 1, K - 16:] = float("inf")
+    d = dict(d, x=x)
+    whole, _ = _run(d, dtype, B, M, K, False, False, out_dtype="f32")
+    whole = whole.reshape(B, M)
+    special = (1, 2, 3, 4, B - 1)
+    for b in special:
+        one, _ = _run(dict(d, x=x[b].contiguous()), dtype, 1, M, K, False, False, out_dtype="f32")
+        assert np.array_equal(np.isnan(one), np.isnan(whole[b])), b
+        inf = np.isinf(one)
+        assert np.array_equal(one[inf], whole[b][inf]) and (inf.any() or b in (3, B - 1)), b
+    rest = [b for b in range(B) if b not in special]
+    hr = dict(h, x=h["x"].reshape(B, K)[rest])
+    err = np.abs(whole[rest].astype(np.float64) - _exact(hr, len(rest), M, K))
+    assert np.all(err <= _bound(hr, len(rest), M, K))
+
+
 @pytest.mark.parametrize("dtype,kv", [("f32", "f32"), ("bf16", "bf16"), ("int8", "bf16"), ("bf16", "int8"),
                                       ("bf16", "fp8"), ("int8", "int8"), ("fp8", "fp8")])
 @pytest.mark.parametrize("B,NH", [(9, 5), (16, 12), (33, 3)])
