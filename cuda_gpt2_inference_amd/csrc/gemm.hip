@@ -539,19 +539,31 @@ bool gemm_takes(int w_dtype, int B, int M, int K) {
     return groups * kGemmWaves * kWave < (1ll << 31);
 }
 
-// The launch for arguments that launch_gemv has checked.  The waves split a row's steps alike
-// whatever the epilogue, so that up to kTallRows rows the QKV projection with the append in its
-// epilogue sums as the plain one does, bit for bit.
+// The launch for arguments that launch_gemv has checked.
 int launch_gemm(GemvArgs a, int w_dtype, bool out_f32, int epi, void* stream) {
     const int wbytes = w_dtype == KVATTN_KV_F32 ? 4 : (w_dtype == KVATTN_KV_BF16 ? 2 : 1);
-    GemmPlan p;
-    switch (w_dtype) {
-        case KVATTN_KV_F32: p = gemm_plan<KVATTN_KV_F32>(a.B, a.M, a.K, out_f32, epi); break;
-        case KVATTN_KV_BF16: p = gemm_plan<KVATTN_KV_BF16>(a.B, a.M, a.K, out_f32, epi); break;
-        case KVATTN_KV_INT8: p = gemm_plan<KVATTN_KV_INT8>(a.B, a.M, a.K, out_f32, epi); break;
-        default: p = gemm_plan<KVATTN_KV_FP8_E4M3>(a.B, a.M, a.K, out_f32, epi); break;
-    }
+    const auto plan = [&](int e) -> GemmPlan {
+        switch (w_dtype) {
+            case KVATTN_KV_F32: return gemm_plan<KVATTN_KV_F32>(a.B, a.M, a.K, out_f32, e);
+            case KVATTN_KV_BF16: return gemm_plan<KVATTN_KV_BF16>(a.B, a.M, a.K, out_f32, e);
+            case KVATTN_KV_INT8: return gemm_plan<KVATTN_KV_INT8>(a.B, a.M, a.K, out_f32, e);
+            default: return gemm_plan<KVATTN_KV_FP8_E4M3>(a.B, a.M, a.K, out_f32, e);
+        }
+    };
+    GemmPlan p = plan(epi);
     if (!p.fn) return KVATTN_ERR_DTYPE;
+    // The QKV projection with the append gives the plain projection's qkv bit for bit: the waves of
+    // gemm_kernel split a row's steps alike whatever the epilogue, and where the plain call keeps
+    // its tokens in LDS (other sums, and no epilogue there), the append is a launch of its own behind it.
+    if (epi != kEpiNone) {
+        const GemmPlan plain = plan(kEpiNone);
+        if (plain.tall && (((uintptr_t)a.out | (uintptr_t)a.kv) & 15u) == 0) {
+            const int st = launch_gemm(a, w_dtype, out_f32, kEpiNone, stream);
+            if (st != KVATTN_OK) return st;
+            return kvattn_cache_write(a.kv, a.kv_scale, a.out, a.B, a.NH, kHd, a.maxT, a.cur_len, a.lens_per_seq,
+                                      a.kv_dtype, stream);
+        }
+    }
     const int steps = (a.K * wbytes / 16 + 3) / 4;
     int col_tiles = (a.B + p.cols - 1) / p.cols;
     int pk_m = a.M | (a.gelu ? kGeluFlag : 0);

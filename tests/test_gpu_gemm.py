@@ -188,6 +188,13 @@ def test_batch_qkv_append_equals_gemv_then_append(dev, dtype, kv, B, NH):
     assert c_b.view(torch.uint8).any()
 
 
+@pytest.mark.parametrize("dtype,kv", [("bf16", "bf16"), ("int8", "bf16"), ("bf16", "int8"), ("fp8", "fp8")])
+@pytest.mark.parametrize("B", [9, 20, 33])
+def test_tall_qkv_append_equals_gemv_then_append(dev, dtype, kv, B):
+    """The same from 20000 rows on (105 heads), where the plain projection keeps its tokens in LDS."""
+    test_batch_qkv_append_equals_gemv_then_append(dev, dtype, kv, B, 105)
+
+
 def test_tall_batch_in_a_graph(dev):
     """The kernel with tokens in LDS (more than 64 KB of it) captured and replayed over new tokens,
     with eager work in between: every replay as the eager call."""
