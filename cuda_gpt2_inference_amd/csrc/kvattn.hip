@@ -3043,7 +3043,7 @@ int kvattn_plan(int B, int NH, int hs, int maxT, int len_hint, int S, int strate
     Plan p{};
     KV_TRY(make_plan(B, NH, maxT, len_hint, S, strategy, kv_dtype, p));
     *strategy_out = p.strategy;
-    *segments_out = p.slots;
+    *segments_out = p.ws_slots > 0 ? p.ws_slots : p.slots;   // what the call's workspace must hold
     *seg_rows_out = p.seg_rows < 0 ? -1 : p.seg_rows;
     return KVATTN_OK;
 }

@@ -299,7 +299,7 @@ def set_merge_poll_limit(polls: int) -> int:
 
 
 def plan(B, NH, hs, maxT, *, kv_dtype, len_hint=-1, S=0, strategy="auto"):
-    """(strategy code, segment slots per (b,h), rows per segment) kvattn_decode would use."""
+    """(strategy code, segment slots per (b,h) its workspace must hold, rows per segment) of kvattn_decode."""
     st, seg, rows = _i(), _i(), _i()
     _check(lib().kvattn_plan(B, NH, hs, maxT, int(len_hint), int(S), strategy_code(strategy),
                              kv_dtype_code(kv_dtype), ctypes.byref(st), ctypes.byref(seg), ctypes.byref(rows)),

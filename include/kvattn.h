@@ -242,10 +242,16 @@ int kvattn_set_xcd_layout_offset(int rot);
 int kvattn_set_merge_poll_limit(int polls);
 
 /* The launch plan kvattn_decode would use for these arguments, without launching:
- * *strategy_out = the resolved kvattn_strategy (AUTO resolved), *segments_out = segment
- * slots per (b,h) (1 for FUSED_SINGLE), *seg_rows_out = rows per segment (0 when the
- * reference partition ceil(total/S) is used, -1 when the kernels plan the rows from the
- * device length).  The plan is that of a call with one length for the batch
+ * *strategy_out = the resolved kvattn_strategy (AUTO resolved), *segments_out = the segment
+ * slots per (b,h) that the call's workspace must hold, so that
+ * kvattn_workspace_bytes(B, NH, hs, maxT, *segments_out) bytes are enough for it,
+ * *seg_rows_out = rows per segment (0 when there are no segments or the reference partition
+ * ceil(total/S) is used, -1 when the kernels plan the rows from the device length).  The slots
+ * are the launch's own (1 for FUSED_SINGLE), except for AUTO's plans for many heads of 257 to
+ * 1024 positions (FUSED_SINGLE, or one segment per (b,h) on an INT8 cache): kvattn_decode asks
+ * for the workspace of the segments that such a plan stands in for, and these are reported.
+ * (FUSED_SINGLE passed by name asks for none.)
+ * The plan is that of a call with one length for the batch
  * (lens_per_seq == 0).  A call with per-sequence lengths takes the same plan, except where
  * this one streams a BF16 or INT8 cache through the split + merge kernels: there AUTO keeps
  * its general plan (the last-block merge, or split + merge over segments of up to 512
@@ -273,8 +279,11 @@ int kvattn_plan(int B, int NH, int hs, int maxT, int len_hint, int S, int strate
  *              lets the library pick the rows per segment (from len_hint, or on the
  *              device) and the per-sequence count from each length.
  *   workspace  device memory of kvattn_workspace_bytes(B, NH, hs, maxT, S) bytes,
- *              initialised once with kvattn_workspace_init; may be NULL for
- *              FUSED_SINGLE.  Calls sharing a workspace must be ordered: on one stream,
+ *              initialised once with kvattn_workspace_init; may be NULL for strategy
+ *              FUSED_SINGLE and for AUTO up to 256 positions (the hint's, else maxT).
+ *              AUTO's plans for many heads beyond that ask for a workspace also where the
+ *              launch uses less of it or none (kvattn_plan reports its slots).
+ *              Calls sharing a workspace must be ordered: on one stream,
  *              or on several streams ordered by events (the designated merger's words
  *              carry the dispatch and its hardware queue, so a word another stream's call
  *              left is never taken for this call's).  Calls that overlap in time race.
@@ -298,8 +307,10 @@ int kvattn_decode(void* out, const void* qkv, const void* kv_cache, const float*
  * a fill kernel clears the array's counters on its first call on a device).
  * No reference counterpart: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * Limits: B*NH <= 16384, and the plan's partials and tagged words (kvattn_workspace_bytes
- * less its status words and counters) within 8 MiB - 64.25 KiB, else KVATTN_ERR_WORKSPACE;
+ * Limits: B*NH <= 16384, and the plan's partials and tagged words (kvattn_workspace_bytes of
+ * the slots that kvattn_plan reports, less its status words and counters) within
+ * 8 MiB - 64.25 KiB, else KVATTN_ERR_WORKSPACE (AUTO falls back on segments that fit where it
+ * can; its plans for many heads are refused with the segments that they stand in for);
  * strategies AUTO, FUSED_SINGLE, SPLIT_MERGE, SPLIT_LASTBLOCK, SPLIT_DESIGNATED (the
  * cooperative launch and the library's graph pair return KVATTN_ERR_STRATEGY: the runtime may
  * allocate for them).  Every call on one GPU shares that GPU's array (with

@@ -101,3 +101,38 @@ def test_many_heads_accept_the_replaced_plans_workspace(dev):
     with pytest.raises(kvattn.KvAttnError) as e:
         kvattn.decode(out, qkv, cache, B, NH, HS, maxT, workspace=ws, workspace_nbytes=n - 4096, **kw)
     assert e.value.status == kvattn.ERR_WORKSPACE
+
+
+@pytest.mark.parametrize("dtype,B,NH,maxT,hint", [
+    ("bf16", 48, 12, 700, -1), ("bf16", 48, 12, 700, 699), ("bf16", 64, 12, 1024, 1023), ("bf16", 40, 12, 2048, 600),
+    ("fp8", 24, 10, 512, 299), ("fp8", 64, 12, 700, -1), ("fp8", 60, 8, 1024, 1023), ("f32", 60, 12, 700, 699),
+    ("f32", 64, 12, 1024, 1023), ("int8", 40, 12, 1024, -1), ("int8", 96, 12, 700, 600)])
+def test_the_reported_slots_are_workspace_enough(dev, dtype, B, NH, maxT, hint):
+    """kvattn_workspace_bytes of the slots that kvattn_plan reports is what AUTO asks for: accepted,
+    and refused with one slot less; fused_single by name asks for none."""
+    import torch
+    from cuda_gpt2_inference_amd import kvattn
+    strategy, slots, _ = kvattn.plan(B, NH, HS, maxT, kv_dtype=dtype, len_hint=hint)
+    assert strategy == (kvattn.SPLIT_LASTBLOCK if dtype == "int8" else kvattn.FUSED_SINGLE)
+    act = torch.float32 if dtype == "f32" else torch.bfloat16
+    w8 = dtype in ("int8", "fp8")
+    cache = torch.zeros(2, B, NH, maxT, HS, dtype=torch.uint8 if w8 else act, device=dev)
+    scale = torch.ones(2, B, NH, maxT, device=dev) if w8 else None
+    qkv = torch.ones(B, 3, NH, HS, dtype=act, device=dev)
+    out = torch.full((B, NH, HS), float("nan"), dtype=act, device=dev)
+    cur = torch.tensor([hint if hint >= 0 else maxT - 1], dtype=torch.int32, device=dev)
+    kw = dict(kv_dtype=dtype, kv_scale=scale, cur_len=cur, len_hint=hint)
+    n = kvattn.workspace_bytes(B, NH, HS, maxT, slots)
+    ws = torch.zeros(n, dtype=torch.uint8, device=dev)
+    kvattn.decode(out, qkv, cache, B, NH, HS, maxT, workspace=ws, workspace_nbytes=n, **kw)
+    torch.cuda.synchronize()
+    assert not out.any()
+    if strategy == kvattn.FUSED_SINGLE:
+        kvattn.decode(out.fill_(float("nan")), qkv, cache, B, NH, HS, maxT, strategy=strategy, **kw)
+        torch.cuda.synchronize()
+        assert not out.any()
+    if slots > 1:
+        less = kvattn.workspace_bytes(B, NH, HS, maxT, slots - 1)
+        with pytest.raises(kvattn.KvAttnError) as e:
+            kvattn.decode(out, qkv, cache, B, NH, HS, maxT, workspace=ws, workspace_nbytes=less, **kw)
+        assert e.value.status == kvattn.ERR_WORKSPACE
