@@ -514,24 +514,43 @@ GemmPlan gemm_plan(int B, int M, int K, bool out_f32, int epi) {
 
 namespace kvattn_internal {
 
-// Whether a call takes the matrix cores.  Measured, gemv.hip / this file (us per call, graph of
-// calls, MI355X; rows x K, tokens):
-//   BF16  768 x 768    2: 2.8 / 2.9   3: 3.7 / 2.9   768 x 3072  4: 4.8 / 5.1   5: 5.3 / 5.1
-//   FP8   768 x 768    2: 2.5 / 2.7   768 x 3072  2: 3.4 / 4.3   4: 4.4 / 4.3
-//   INT8  768 x 3072   2: 3.2 / 4.6   3: 3.5 / 4.6
-//   FP32  768 x 768    5: 3.9 / 4.3   7: 4.7 / 4.3   768 x 3072  5: 6.4 / 10.5  7: 7.5 / 11.9
-//         1280 x 5120  4: 28.6 / 20.1 (gemv.hip takes rows this long in blocks)
-// So from 3 tokens on.  Few rows (at most 1024: 64 tiles here) of more than 1600 but still one block
-// of gemv.hip leave most of the chip idle here, and stay there for 2 (8-bit weights: 1) tokens
-// more.  FP32 weights, whose MFMA does a sixteenth of the work: 4; few rows up to 1024 long 6; 8
-// beyond 1600, few 12.
+// Whether a call takes the matrix cores: from how many vectors on.  us per call, gemv.hip / this
+// file (graph of calls, MI355X; vectors : us):
+//   BF16   768 x   768   2: 3.1 / 3.0    3: 3.5 / 3.0      768 x  3072   4: 5.0 / 5.3    5: 5.5 / 5.3
+//         1024 x  5120   3: 6.8 / 7.4    4: 7.8 / 7.4      256 x  8192   4: 9.1 / 10.2   5: 10.6 / 10.3
+//          256 x 12288   3: 16.0 / 13.8                    512 x 32768   3: 32.3 / 38.5  4: 41.7 / 39.4
+//   INT8   768 x   768   2: 2.9 / 3.0    3: 3.3 / 3.0      768 x  2048   3: 3.7 / 3.9    4: 4.1 / 3.9
+//          768 x  8192   4: 8.3 / 9.2    5: 9.4 / 9.2      768 x 16384   4: 14.9 / 15.5  5: 17.5 / 15.5
+//          768 x 20000   3: 23.9 / 18.1                    768 x 32768   3: 25.6 / 27.5  4: 32.7 / 27.6
+//   FP8    256 x  3072   3: 3.8 / 4.1    4: 4.3 / 4.1      256 x 16384   4: 12.9 / 13.2  5: 15.5 / 13.3
+//   FP32   768 x   320   4: 3.6 / 3.0    5: 4.0 / 3.0      768 x  1024   5: 4.4 / 5.3    7: 5.1 / 5.3
+//         1024 x  1600   7: 6.4 / 6.6    8: 6.9 / 6.6      768 x  3072  11: 10.0 / 10.7 12: 10.6 / 10.7
+//         1280 x  1024   4: 4.6 / 5.4    5: 5.0 / 5.4     1280 x  1600   4: 6.3 / 6.7    5: 6.8 / 6.6
+//         3072 x   768   3: 4.9 / 4.9    4: 5.3 / 4.8     2048 x  4096   7: 16.1 / 16.6  8: 17.2 / 16.6
+//         1280 x  4096   8: 15.6 / 17.1
+//         1024 x  5120   3: 15.9 / 20.0  4: 19.8 / 20.0    256 x  6144   4: 18.1 / 18.9  5: 21.7 / 18.9
+//          512 x  8192   5: 25.0 / 26.2  6: 29.4 / 26.7    512 x 16384   5: 47.6 / 53.6  6: 56.6 / 54.5
+// The vector units' time grows with the vectors, this file's hardly does: from 3 on.  Few rows (up
+// to 1024: 64 tiles here) that are long, but still one block of gemv.hip (16 KB), leave most of
+// the chip idle here while that kernel keeps the weights in registers: 4 or 5.  Beyond a block
+// gemv.hip reads the weights again for every vector: 3, from two blocks on 4.  FP32 weights, whose MFMA
+// does a sixteenth of the work, come later throughout, and latest for few rows of up to one block.
 bool gemm_takes(int w_dtype, int B, int M, int K) {
-    const bool few = M <= 1024, mid = K > 1600 && K <= 4096;
+    const bool few = M <= 1024;
     int from = 3;
-    switch (w_dtype) {
-        case KVATTN_KV_F32: from = mid ? (few ? 12 : 8) : (few && K <= 1024 ? 6 : 4); break;
-        case KVATTN_KV_BF16: from = few && mid ? 5 : 3; break;
-        default: from = few && mid ? 4 : 3; break;
+    if (w_dtype == KVATTN_KV_F32) {
+        const bool mid = M <= 1536;
+        if (K <= 768) from = few ? 6 : 4;
+        else if (K <= 1024) from = few ? 6 : (mid ? 5 : 4);
+        else if (K <= 1600) from = few ? 8 : (mid ? 5 : 4);
+        else if (K <= 4096) from = few ? 12 : (M <= 1280 && K > 3072 ? 9 : 8);
+        else if (few) from = K <= 5120 ? 4 : (K <= 6144 ? 5 : 6);
+        else from = 4;
+    } else if (few && K > 1600) {
+        const int row = w_dtype == KVATTN_KV_BF16 ? 2 * K : K;
+        if (row > 16384) from = row < 32768 ? 3 : 4;
+        else if (w_dtype == KVATTN_KV_BF16) from = K > 4096 && K <= 6144 ? 4 : 5;
+        else from = K <= 6144 ? 4 : 5;
     }
     if (B < from || K > (1 << 20)) return false;
     // Grids beyond 2^31 threads stay with gemv.hip.

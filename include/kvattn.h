@@ -382,14 +382,18 @@ int kvattn_paged_decode(void* out, const void* qkv, void* pages, float* page_sca
  *              out, pre_gelu bf16
  * W is row-major [M][K]; x [B][K]; out [B][M].  Requires K % 16 == 0 (any length: rows
  * beyond 64 * 16 chunks of 16 bytes are walked in blocks, as the reference's tail loops walk
- * any K), 16-byte aligned W and x.  bias may be NULL.  From 8192 rows on (a vocabulary
- * projection), each wave takes 4 rows so that more weight bytes are in flight.
+ * any K), 16-byte aligned W and x.  bias may be NULL.  One or two vectors (and few vectors
+ * where the matrix cores do not pay) take one wave per row; from 8192 rows on (a vocabulary
+ * projection) a wave takes 4 rows of 8-bit weights, 2 of wider ones, so that more weight
+ * bytes are in flight.
  * Replaces launch_GEMV6_fused (Inference_gpt2/GEMV.cuh:132-206) and launch_GEMV6_w8x2
  * (Inference_gpt2/GEMV_w8.cuh:64-184), which matmul_forward[_w8] calls for one decode token
  * (inference_gpt2_opt.cu:106-132); the attention output projection is at :349-355.  Batches
- * (from 3 vectors on; few long rows 4 or 5, FP32 weights 4 to 12) go through the matrix cores with FP32 sums, where the reference takes cuBLASLt; other B > 1 read the weights once for all B
- * vectors when a row fits in one block.  A vector's result may differ in its last bits with
- * the size of the batch (another order of the same sums). */
+ * (from 3 vectors on; up to 1024 rows of more than 1600 columns from 3 to 5, FP32 weights
+ * from 4 to 12) go through the matrix cores with FP32 sums, where the reference takes
+ * cuBLASLt; other B > 1 read the weights once for all B vectors when a row fits in one
+ * block.  A vector's result may differ in its last bits with the size of the batch (another
+ * order of the same sums). */
 int kvattn_gemv(void* out, void* pre_gelu, const void* W, const float* w_scale, const void* x,
                 const void* bias, int B, int M, int K, int w_dtype, int gelu, void* stream);
 

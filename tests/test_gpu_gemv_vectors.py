@@ -61,3 +61,35 @@ def test_append_of_two_vectors(dev, dtype):
     for b, t in enumerate((3, 15)):
         want[:, b, :, t] = ref[b].view(3, NH, 64)[1:]
     assert torch.equal(cache, want)
+
+
+@pytest.mark.parametrize("dtype,B,M,K", [("f32", 5, 1024, 1024), ("f32", 7, 260, 1040), ("f32", 7, 1024, 1600),
+                                         ("f32", 4, 1280, 1040), ("f32", 11, 37, 4096), ("f32", 4, 200, 6144),
+                                         ("f32", 5, 1024, 12288), ("f32", 4, 1300, 784), ("f32", 8, 1280, 4096),
+                                         ("bf16", 4, 1000, 1616),
+                                         ("bf16", 3, 70, 5136), ("bf16", 4, 256, 8192), ("bf16", 3, 100, 16384),
+                                         ("int8", 3, 512, 4096), ("int8", 4, 768, 8192), ("fp8", 4, 300, 16384),
+                                         ("int8", 3, 64, 32768), ("fp8", 3, 1024, 6144)])
+def test_few_vectors_over_few_long_rows_keep_their_bits(dev, dtype, B, M, K):
+    """Where a few long rows would leave most of the chip idle as matrix-core tiles, every vector is
+    the one it is alone, bit for bit."""
+    import torch
+    from cuda_gpt2_inference_amd import kvattn
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + K)
+    act = torch.float32 if dtype == "f32" else torch.bfloat16
+    x = torch.randn(B, K, generator=g, device=dev).to(act)
+    scale = None
+    if dtype in ("int8", "fp8"):
+        W = torch.randint(0, 120, (M, K), generator=g, device=dev, dtype=torch.uint8)
+        scale = 1e-3 * torch.rand(M, generator=g, device=dev)
+    else:
+        W = torch.randn(M, K, generator=g, device=dev).to(act)
+    kw = dict(w_dtype=dtype, w_scale=scale, out_dtype="f32")
+    got = torch.full((B, M), float("nan"), device=dev)
+    kvattn.gemv(got, W, x, B, M, K, **kw)
+    for b in range(B):
+        one = torch.full((1, M), float("nan"), device=dev)
+        kvattn.gemv(one, W, x[b:b + 1].contiguous(), 1, M, K, **kw)
+        torch.cuda.synchronize()
+        assert torch.isfinite(one).all() and torch.equal(one[0], got[b]), b
