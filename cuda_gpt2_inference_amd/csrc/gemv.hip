@@ -309,6 +309,23 @@ constexpr int kGemvTallRows = KVATTN_GEMV_TALL_ROWS;
 // Most chunks per lane for which the next vector's x fits the registers beside this one's.
 template <int WT> constexpr int kPreMaxChunks = WT == KVATTN_KV_F32 ? 16 : WT == KVATTN_KV_BF16 ? 8 : 4;
 
+// Whether the next vector's x is requested ahead (kPre).  It hides a round trip for every vector
+// while the grid's waves all run at once; a larger grid hides it by itself, and loses waves per
+// SIMD to the registers.  us per call, not ahead / ahead:
+//   FP32  768 x 3072  2:  4.9 /  4.8  7:  8.5 /  7.8   1024 x 4096  2: 6.2 / 6.4  4: 8.2 / 7.8
+//        1536 x 2048  2:  5.4 /  5.4  4:  6.8 /  6.8   2304 x 2048  2: 6.6 / 7.0  4: 8.4 / 8.9
+//        4096 x 4096  2: 16.0 / 20.8  4: 20.7 / 26.4   1280 x 3072  2: 6.6 / 6.7  4: 8.5 / 8.8
+//   BF16, 2 vectors   768 x 3072 4.1 / 3.9   2304 x  768 3.9 /  3.7   3072 x 2048 5.9 / 5.7
+//                    1536 x 4096 6.4 / 6.5   4096 x 4096 10.0 / 10.9  6144 x 2048 8.1 / 8.4
+//   INT8, 2          1280 x 4096 5.2 / 4.9   3072 x 4096 7.1 /  6.8   6144 x 1600 6.6 / 7.0
+//   FP8, 2           3072 x 3072 5.8 / 5.7   4096 x 4096 7.8 /  8.2   6144 x 1600 6.4 / 6.9
+template <int WT>
+bool pre_pays(int M, int lane_chunks, int vectors) {
+    if (vectors < 2 || lane_chunks > kPreMaxChunks<WT>) return false;
+    if (M <= 1024) return vectors > 2 || lane_chunks <= 12;
+    return M <= 4096 && lane_chunks <= (WT == KVATTN_KV_F32 ? 8 : 6) && M * lane_chunks <= 12288;
+}
+
 // One row per wave.  3, 6 and 12 chunks beside the powers of two: a lane's chunks beyond the row are
 // loaded and multiplied for nothing (768 x 3072, one vector, 8 / 6 chunks BF16 3.56 / 3.25 us, 4 / 3
 // FP8 3.11 / 2.95, 16 / 12 FP32 4.17 / 4.04).
@@ -331,7 +348,7 @@ const void* gemv_row_ptr(int chunks_per_lane) {
 }
 
 template <int WT, bool kOut, int kEpi>
-const void* gemv_ptr(int chunks_per_lane, int rows, int vectors) {
+const void* gemv_ptr(int M, int chunks_per_lane, int rows, int vectors) {
     if constexpr (kEpi == kEpiNone) {
         if constexpr (WFmt<WT>::k8bit) {
             if (rows == 4) {
@@ -347,23 +364,22 @@ const void* gemv_ptr(int chunks_per_lane, int rows, int vectors) {
         }
     }
     if constexpr (kEpi != kEpiAppend8)
-        if (vectors > 1 && chunks_per_lane <= kPreMaxChunks<WT>)
-            return gemv_row_ptr<WT, kOut, kEpi, true>(chunks_per_lane);
+        if (pre_pays<WT>(M, chunks_per_lane, vectors)) return gemv_row_ptr<WT, kOut, kEpi, true>(chunks_per_lane);
     return gemv_row_ptr<WT, kOut, kEpi, false>(chunks_per_lane);
 }
 
 // The QKV epilogue writes qkv in the activation type, so only the plain GEMV takes another
 // output type.
 template <int WT>
-const void* gemv_ptr_out(int chunks_per_lane, int rows, int vectors, bool out_f32, int epi) {
+const void* gemv_ptr_out(int M, int chunks_per_lane, int rows, int vectors, bool out_f32, int epi) {
     constexpr bool kAct = WFmt<WT>::kActF32;
-    if (epi == kEpiAppend) return gemv_ptr<WT, kAct, kEpiAppend>(chunks_per_lane, 1, vectors);
+    if (epi == kEpiAppend) return gemv_ptr<WT, kAct, kEpiAppend>(M, chunks_per_lane, 1, vectors);
     if (epi == kEpiAppend8) {
         if constexpr (kAct) return nullptr;   // 8-bit caches sit behind bf16 activations
-        else return gemv_ptr<WT, false, kEpiAppend8>(chunks_per_lane, 1, vectors);
+        else return gemv_ptr<WT, false, kEpiAppend8>(M, chunks_per_lane, 1, vectors);
     }
-    return out_f32 ? gemv_ptr<WT, true, kEpiNone>(chunks_per_lane, rows, vectors)
-                   : gemv_ptr<WT, false, kEpiNone>(chunks_per_lane, rows, vectors);
+    return out_f32 ? gemv_ptr<WT, true, kEpiNone>(M, chunks_per_lane, rows, vectors)
+                   : gemv_ptr<WT, false, kEpiNone>(M, chunks_per_lane, rows, vectors);
 }
 
 }  // namespace
@@ -403,10 +419,10 @@ int launch_gemv(GemvArgs a, int w_dtype, bool out_f32, void* stream) {
     const int rows = a.kv || M < kGemvTallRows ? 1 : (w8 ? 4 : 2);
     const void* fn = nullptr;
     switch (w_dtype) {
-        case KVATTN_KV_F32: fn = gemv_ptr_out<KVATTN_KV_F32>(per_lane, rows, B, out_f32, epi); break;
-        case KVATTN_KV_BF16: fn = gemv_ptr_out<KVATTN_KV_BF16>(per_lane, rows, B, out_f32, epi); break;
-        case KVATTN_KV_INT8: fn = gemv_ptr_out<KVATTN_KV_INT8>(per_lane, rows, B, out_f32, epi); break;
-        default: fn = gemv_ptr_out<KVATTN_KV_FP8_E4M3>(per_lane, rows, B, out_f32, epi); break;
+        case KVATTN_KV_F32: fn = gemv_ptr_out<KVATTN_KV_F32>(M, per_lane, rows, B, out_f32, epi); break;
+        case KVATTN_KV_BF16: fn = gemv_ptr_out<KVATTN_KV_BF16>(M, per_lane, rows, B, out_f32, epi); break;
+        case KVATTN_KV_INT8: fn = gemv_ptr_out<KVATTN_KV_INT8>(M, per_lane, rows, B, out_f32, epi); break;
+        default: fn = gemv_ptr_out<KVATTN_KV_FP8_E4M3>(M, per_lane, rows, B, out_f32, epi); break;
     }
     if (!fn) return KVATTN_ERR_DTYPE;
     long long groups = ((M + rows - 1) / rows + kGemvWaves - 1) / kGemvWaves;

@@ -38,6 +38,33 @@ def test_vectors_are_those_of_single_calls(dev, dtype, lane_chunks, edge):
             assert torch.isfinite(o).all() and torch.equal(o[0], w[b])
 
 
+@pytest.mark.parametrize("dtype,B,K", [("f32", 3, 1024), ("f32", 2, 2048), ("f32", 2, 4096), ("bf16", 2, 3072),
+                                       ("bf16", 2, 2048), ("int8", 2, 4096), ("fp8", 2, 1040)])
+@pytest.mark.parametrize("M", [1024, 1025, 1536, 1537, 3073, 4096, 4097])
+def test_vectors_keep_their_bits_at_every_height(dev, dtype, B, K, M):
+    """On either side of the heights up to which the next vector's x is requested ahead."""
+    import torch
+    from cuda_gpt2_inference_amd import kvattn
+    g = torch.Generator(device=dev)
+    g.manual_seed(K + M)
+    act = torch.float32 if dtype == "f32" else torch.bfloat16
+    x = torch.randn(B, K, generator=g, device=dev).to(act)
+    scale = None
+    if dtype in ("int8", "fp8"):
+        W = torch.randint(0, 120, (M, K), generator=g, device=dev, dtype=torch.uint8)
+        scale = 1e-3 * torch.rand(M, generator=g, device=dev)
+    else:
+        W = torch.randn(M, K, generator=g, device=dev).to(act)
+    kw = dict(w_dtype=dtype, w_scale=scale, out_dtype="f32")
+    got = torch.full((B, M), float("nan"), device=dev)
+    kvattn.gemv(got, W, x, B, M, K, **kw)
+    for b in range(B):
+        one = torch.full((1, M), float("nan"), device=dev)
+        kvattn.gemv(one, W, x[b:b + 1].contiguous(), 1, M, K, **kw)
+        torch.cuda.synchronize()
+        assert torch.isfinite(one).all() and torch.equal(one[0], got[b]), b
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_append_of_two_vectors(dev, dtype):
     import torch
