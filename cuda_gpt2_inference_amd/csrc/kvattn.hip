@@ -2354,9 +2354,12 @@ bool latency_bound(int B, int NH, int total_rows, bool ragged = false, bool k8 =
 // only its first two cases).
 // - One segment per (b,h) (last-block instance, which then stores without a merge) when the
 //   heads alone give 192 or more workgroups and no head is longer than 512 rows; 8-bit caches
-//   take the streaming shape's 64-row tiles there below 384 heads and from 1024 on (INT8, us per
-//   call, streaming / latency shape: 240 heads of 300 positions 6.52 / 6.76, 576 of 300 10.13 /
-//   9.24, 1536 of 400 18.2 / 19.4, 1152 of 1024 30.0 / 32.4).
+//   take the streaming shape's 64-row tiles there, contiguous INT8 ones of known length (a hint, or
+//   every one of up to kOneSegLatSeqs sequences its own) the latency shape's from kOneSegLatHeads to
+//   1023 heads (us per call, streaming / latency: 384 heads of 512 positions 7.84 / 8.12, 480 of 400 7.72 / 8.18; 576
+//   of 300 8.87 / 8.83, of 400 9.63 / 9.52, U[1, 512] 9.98 / 9.30, 640 sequences of one head 14.0 / 15.6; 768 of 300 9.90 / 9.43; 1536 of
+//   400 18.2 / 19.4.  Without a hint a graph meets every length, and 129 to 255 positions lose what
+//   shorter ones gain: 768 heads, maxT 512, of 100 6.58 / 5.47, of 200 7.21 / 8.16).
 // - The designated merger while its grid stays within kAutoDesignatedMaxGrid workgroups and
 //   the call streams at most kAutoDesignatedMaxBytes: segments of max(128, maxT / 16) rows
 //   (a power of two, so at most 16 per head; up to 64 per head when fewer than 12 heads
@@ -2379,10 +2382,13 @@ bool latency_bound(int B, int NH, int total_rows, bool ragged = false, bool k8 =
 //   positions ran 9 % slower on 256-row segments), keep the general plan (false).
 // Returns false to leave the plan to the general rules below.
 constexpr long long kManyHeads = 480;
+constexpr long long kOneSegLatHeads = 560;
+constexpr int kOneSegLatSeqs = 256;
 constexpr long long kAutoDesignatedMaxGrid = 768;
 constexpr long long kAutoDesignatedMaxBytes = 64ll << 20;
 constexpr long long kAutoDoubledMaxBytes = 40ll << 20;
-bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragged, bool paged, Plan& p) {
+// known: the host knows the longest length, or every sequence has its own.
+bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragged, bool paged, bool known, Plan& p) {
     const long long heads = (long long)B * NH;
     const bool k8 = is_8bit(kv_dtype);
     const long long row_bytes = kv_dtype == KVATTN_KV_F32 ? 512 : (kv_dtype == KVATTN_KV_BF16 ? 256 : 136);
@@ -2391,7 +2397,8 @@ bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragg
         p.strategy = KVATTN_SPLIT_LASTBLOCK;
         p.seg_rows = 512;
         p.slots = 1;
-        p.lat = !k8 || (!paged && heads >= 384 && heads < 1024);
+        p.lat = !k8 || (kv_dtype == KVATTN_KV_INT8 && !paged && known && heads >= kOneSegLatHeads && heads < 1024 &&
+                        !(ragged && B > kOneSegLatSeqs));
         return true;
     }
     // At most 16 segments per head once the heads give 192 workgroups with them; fewer heads
@@ -2431,32 +2438,47 @@ bool tuned_auto(int B, int NH, int maxT, int total_hint, int kv_dtype, bool ragg
 
 // Many heads of up to 1024 positions fill the GPU by themselves: a workgroup a head, scores in LDS
 // (fused_single), saves the segments' partials and merge, and the second pass over the scores
-// costs less than an online softmax's rescaling.  us per call, a plan of segments / fused_single
-// (NH = 12, the plan made for the longest length; sequences x positions, u: all of that length,
-// r: U[1, that]):
-//   BF16  20 x 300 r 6.94 / 6.36, u 7.49 / 7.60   32 x 300 r 8.17 / 8.01, u 8.70 / 8.67   48 x 300 u 11.3 / 10.4
-//         40 x 700 u 18.9 / 16.1   48 x 1024 u 28.2 / 28.2, r 19.6 / 18.1   64 x 1024 u 35.2 / 32.4, r 23.2 / 21.0
-//         32 x 1024 r 13.18 / 13.19
-//   FP8   20 x 300 r 6.47 / 5.50   64 x 600 u 19.1 / 13.4   64 x 1024 u 21.1 / 18.4, r 16.6 / 13.9
-//         32 x 1024 r  9.89 / 11.48
-//   FP32  40 x 700 u 33.9 / 28.6   48 x 1024 r 30.2 / 31.9   64 x 1024 u 67.0 / 63.3   48 x 300 u 17.7 / 21.0
+// costs less than an online softmax's rescaling.  Returns whether the plan p, made without this
+// rule, is replaced.  known: the host knows the longest length, or every sequence has its own.
+// us per call, a plan of segments / fused_single (NH = 12, the plan made for the longest length;
+// sequences x positions, u: all of that length, r: U[1, that]; "of 2048": hinted, in a cache of 2048):
+//   BF16  40 x  700 u 18.9 / 16.1   48 x 1024 u 28.2 / 28.2, r 19.6 / 18.1   64 x 1024 u 35.2 / 32.4, r 23.2 / 21.0
+//         32 x 1024 r 13.18 / 13.19   32 x  400 u of 1024 10.9 / 10.8
+//     from 321 to 512 positions the passes take a second, partial round of tiles, and caches of up to
+//     512 have one segment per head to lose against, also at the short lengths that a graph without a hint meets:
+//         32 x  400 u 10.11 / 10.21, r 8.41 / 9.85   85 x 400 u 19.6 / 22.2   64 x 17 of 512 5.88 / 6.49
+//         fused_single's time over the segments': r 32 x 290 0.98, 40 x 320 1.02, 48 x 290 0.95, 64 x 320 0.96,
+//         128 x 290 0.92; r of 640 40 x 360 1.07, 48 x 400 0.94
+//   FP8   20 x  300 u 6.48 / 5.86, r 6.39 / 5.73    48 x 300 u  9.63 / 8.27    64 x 600 u 19.1 / 13.4
+//         64 x 1024 u 21.1 / 18.4, r 16.6 / 13.9    32 x 1024 r 9.89 / 11.48
+//     from 321 to 512 positions as above:
+//         20 x  400 u 6.37 / 7.78, r 6.69 / 7.53    40 x 400 u 8.09 / 8.97    48 x 400 u 9.89 / 9.81
+//         over the segments': r 56 x 384 1.07, 64 x 400 1.01, 85 x 400 0.91; of 1024 u 20 x 400 1.07, 25 x 400 0.98,
+//         r 40 x 360 1.03, 48 x 400 0.94; of 2048 u 20 x 400 0.54, r 20 x 400 1.10, 25 x 400 0.94
+//   FP32  40 x  700 u 33.9 / 28.6   48 x 1024 r 30.2 / 31.9   64 x 1024 u 67.0 / 63.3   48 x 300 u 17.7 / 21.0
 //   INT8  48 x 1024 r 14.9 / 20.7 (twice the instructions per byte): one segment per head instead
 //         (last-block instance), 14.2; 40 x 700 u 15.8 / 12.1 in one segment; 64 x 1024 u 21.6 / 19.7
-// Returns whether the plan p, made without this rule, is replaced.
-// known: the host knows the longest length, or every sequence has its own.  (One unknown length for
-// all of up to 769-1024 BF16 positions keeps its device-planned segments: 576 heads u 28.2 / 28.2,
-// 1152 50.9 / 48.9.)
-// FP8 up to 512 positions and FP32 beyond 768 differ with ragged (every sequence its own length): 128 x 400
-// FP8 u 17.3 / 17.8, r 15.2 / 14.1; FP32 56 x 1024 u 60.6 / 57.3, 64 x 1024 r 42.9 / 44.5, 96 x 1024 r 53.2 / 51.8.
+// One unknown length for all of up to 769-1024 BF16 positions keeps its device-planned segments (576
+// heads u 28.2 / 28.2, 1152 50.9 / 48.9).  One-length FP8 up to 512 positions keeps the old plan from 1024
+// heads (128 x 400 u 17.3 / 17.8, r 15.2 / 14.1), FP32 beyond 768 takes this one from 640 or, ragged, 1024
+// (56 x 1024 u 60.6 / 57.3, 64 x 1024 r 42.9 / 44.5, 96 x 1024 r 53.2 / 51.8).
 bool many_heads(long long heads, int maxT, int total, int kv_dtype, bool known, bool ragged, Plan& p) {
     bool fused = total <= 1024 && maxT <= 2048;
     switch (kv_dtype) {
         case KVATTN_KV_BF16:
-            fused = fused && heads >= (total <= 512 ? 384 : kManyHeads) && (known || total <= 768);
+            if (maxT <= 512) fused = fused && ragged && total <= 320 && heads >= 560;
+            else if (total <= 512) fused = fused && heads >= (ragged && total > 320 && maxT <= 1024 ? 560 : 384);
+            else fused = fused && heads >= kManyHeads && (known || total <= 768);
             break;
-        case KVATTN_KV_FP8_E4M3:
-            fused = fused && (total > 512 ? heads >= kManyHeads : heads >= 240 && (ragged || heads < 1024));
+        case KVATTN_KV_FP8_E4M3: {
+            long long from = kManyHeads;
+            if (total <= 320) from = 240;
+            else if (total <= 512 && maxT > 1024) from = ragged ? 300 : 240;
+            else if (total <= 512 && maxT > 512) from = ragged ? 560 : 300;
+            else if (total <= 512) from = ragged ? 960 : 560;
+            fused = fused && heads >= from && (ragged || total > 512 || heads < 1024);
             break;
+        }
         case KVATTN_KV_F32:
             fused = fused && total > 512 && heads >= (total <= 768 ? kManyHeads : ragged ? 1024 : 640);
             break;
@@ -2511,7 +2533,7 @@ int make_plan(int B, int NH, int maxT, int len_hint, int S, int strategy, int kv
             // hinted lengths too, and segments longer than a paged wave walks).
             if (hinted || heads > 16 || heads * designated_slots(maxT, B * NH) > kDesignatedMaxGrid) {
                 Plan q{};
-                if (tuned_auto(B, NH, maxT, hinted ? total_hint : maxT, kv_dtype, ragged, paged, q) &&
+                if (tuned_auto(B, NH, maxT, hinted ? total_hint : maxT, kv_dtype, ragged, paged, ragged || hinted, q) &&
                     (q.strategy != KVATTN_SPLIT_MERGE || (hinted && !paged)) &&
                     !(paged && q.seg_rows > kMaxPagedSegRows)) {
                     p = q;

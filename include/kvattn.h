@@ -253,9 +253,11 @@ int kvattn_set_merge_poll_limit(int polls);
  * (FUSED_SINGLE passed by name asks for none.)
  * The plan is that of a call with one length for the batch
  * (lens_per_seq == 0).  A call with per-sequence lengths takes the same plan, except where
- * this one streams a BF16 or INT8 cache through the split + merge kernels: there AUTO keeps
- * its general plan (the last-block merge, or split + merge over segments of up to 512
- * rows).  No reference counterpart: it exposes the AUTO choice, which the reference makes
+ * this one streams a BF16 or INT8 cache through the split + merge kernels (there AUTO keeps
+ * its general plan: the last-block merge, or split + merge over segments of up to 512
+ * rows), and for many heads of 257 to 1024 positions, whose bounds on the heads differ.  Its
+ * workspace may then differ from the reported one too: S == 0 in kvattn_workspace_bytes is
+ * enough for every call.  No reference counterpart: it exposes the AUTO choice, which the reference makes
  * inline in its caller (inference_gpt2_opt.cu:247,304,331: fused_single below a length
  * threshold, split + merge above it). */
 int kvattn_plan(int B, int NH, int hs, int maxT, int len_hint, int S, int strategy, int kv_dtype,

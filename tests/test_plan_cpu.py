@@ -252,3 +252,44 @@ def test_auto_caps_hinted_split_segments_at_64_per_head():
     # covering maxT
     assert kvattn.plan(8, 12, 64, 65536, kv_dtype="bf16", len_hint=16383) == (kvattn.SPLIT_MERGE, 256, 256)
     assert kvattn.plan(4, 12, 64, 32768, kv_dtype="fp8", len_hint=32767) == (kvattn.SPLIT_MERGE, 64, 512)
+
+
+# (B, NH, maxT, hint, dtype) -> AUTO's strategy and rows per segment, on either side of the edges of
+# the rule for many heads of up to 1024 positions.
+MANY_HEADS = [
+    ((40, 12, 512, -1, "bf16"), (kvattn.SPLIT_LASTBLOCK, 512)),     # caches of up to 512: one segment
+    ((85, 12, 400, 399, "bf16"), (kvattn.SPLIT_LASTBLOCK, 512)),
+    ((64, 12, 300, 299, "bf16"), (kvattn.SPLIT_LASTBLOCK, 512)),
+    ((32, 12, 513, 299, "bf16"), (kvattn.FUSED_SINGLE, 0)),         # longer caches: 384 heads up to 512
+    ((32, 12, 1024, 511, "bf16"), (kvattn.FUSED_SINGLE, 0)),
+    ((383, 1, 1024, 511, "bf16"), (kvattn.SPLIT_DESIGNATED, 512)),
+    ((40, 12, 1024, 512, "bf16"), (kvattn.FUSED_SINGLE, 0)),        # 480 heads beyond
+    ((479, 1, 1024, 512, "bf16"), (kvattn.SPLIT_MERGE, 256)),
+    ((40, 12, 1024, 1023, "bf16"), (kvattn.FUSED_SINGLE, 0)),
+    ((40, 12, 1025, 1024, "bf16"), (kvattn.SPLIT_MERGE, 256)),
+    ((40, 12, 768, -1, "bf16"), (kvattn.FUSED_SINGLE, 0)),          # one unknown length: up to 768
+    ((40, 12, 769, -1, "bf16"), (kvattn.SPLIT_LASTBLOCK, -1)),
+    ((20, 12, 512, 319, "fp8"), (kvattn.FUSED_SINGLE, 0)),          # 240 heads up to 320 positions
+    ((239, 1, 512, 319, "fp8"), (kvattn.SPLIT_LASTBLOCK, 512)),
+    ((20, 12, 512, 320, "fp8"), (kvattn.SPLIT_LASTBLOCK, 512)),
+    ((20, 12, 512, -1, "fp8"), (kvattn.SPLIT_LASTBLOCK, 512)),
+    ((559, 1, 512, -1, "fp8"), (kvattn.SPLIT_LASTBLOCK, 512)),      # 560 up to 512
+    ((560, 1, 512, -1, "fp8"), (kvattn.FUSED_SINGLE, 0)),
+    ((1024, 1, 512, 511, "fp8"), (kvattn.SPLIT_LASTBLOCK, 512)),    # below 1024
+    ((25, 12, 1024, 399, "fp8"), (kvattn.FUSED_SINGLE, 0)),         # 300 of a longer cache
+    ((20, 12, 2048, 399, "fp8"), (kvattn.FUSED_SINGLE, 0)),         # 240 of one beyond 1024
+    ((40, 12, 1024, 1023, "fp8"), (kvattn.FUSED_SINGLE, 0)),
+    ((40, 12, 768, 767, "f32"), (kvattn.FUSED_SINGLE, 0)),
+    ((40, 12, 1024, 1023, "f32"), (kvattn.SPLIT_LASTBLOCK, 256)),
+    ((640, 1, 1024, 1023, "f32"), (kvattn.FUSED_SINGLE, 0)),
+    ((64, 12, 512, 511, "f32"), (kvattn.SPLIT_LASTBLOCK, 512)),
+    ((40, 12, 513, -1, "int8"), (kvattn.SPLIT_LASTBLOCK, 1024)),
+    ((40, 12, 512, -1, "int8"), (kvattn.SPLIT_LASTBLOCK, 512)),
+]
+
+
+@pytest.mark.parametrize("args,plan", MANY_HEADS, ids=["-".join(map(str, a)) for a, _ in MANY_HEADS])
+def test_auto_many_heads_edges(args, plan):
+    B, NH, maxT, hint, dt = args
+    strategy, _, rows = kvattn.plan(B, NH, 64, maxT, kv_dtype=dt, len_hint=hint)
+    assert (strategy, rows) == plan
