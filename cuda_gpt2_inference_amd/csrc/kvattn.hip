@@ -174,7 +174,12 @@ __device__ __forceinline__ float dot_chunk(const float (&q)[Row<DT>::kElems], co
         s = __builtin_amdgcn_fdot2_f32_bf16(pair(d.y), qp(1), s, false);
         s = __builtin_amdgcn_fdot2_f32_bf16(pair(d.z), qp(2), s, false);
         s = __builtin_amdgcn_fdot2_f32_bf16(pair(d.w), qp(3), s, false);
-        return s * q[4];
+        // The lanes of a row add these up: fused into that sum, each lane would round its own product
+        // differently, and they would hold different scores.
+        {
+#pragma clang fp contract(off)
+            return s * q[4];
+        }
     } else {
         float x[Row<DT>::kElems];
         decode<DT>(d, x);
@@ -183,6 +188,14 @@ __device__ __forceinline__ float dot_chunk(const float (&q)[Row<DT>::kElems], co
         for (int e = 0; e < Row<DT>::kElems; ++e) s = fmaf(q[e], x[e], s);
         return s;
     }
+}
+
+// A score's distance from the maximum, of scores as they were compared: fused with the product
+// that made the score (an 8-bit row's scale), the largest score's would be its rounding error,
+// which is no longer zero but beyond exp2's range once scores reach 2^31.
+__device__ __forceinline__ float below_max(float score, float max) {
+#pragma clang fp contract(off)
+    return score - max;
 }
 
 // Attended positions of sequence b: device length clamped to [0, maxT-1], plus one.
@@ -475,7 +488,7 @@ __device__ __forceinline__ void consume_tile(const Tile<DT, U>& t, int r, int r1
     for (int e = 0; e < R::kElems; ++e) acc[e] *= corr;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const float p = exp2_fast(s[u] - mt);
+        const float p = exp2_fast(below_max(s[u], mt));
         l += p;
         const bool live = !kChecked || r + u * kRPL + slot_row < r1;
         const uint4 vd = live ? t.v[u] : make_uint4(0u, 0u, 0u, 0u);
@@ -717,7 +730,7 @@ __device__ __forceinline__ void weight_tile(const Slot& sl, int r, int total, in
     for (int u = 0; u < U; ++u) {
         const int row = r + u * kRPL + slot_row;
         if (!kChecked || row < total) {
-            const float p = exp2_fast(scores[row] - M);
+            const float p = exp2_fast(below_max(scores[row], M));
             l += p;
             const float pv = R::k8bit ? p * vs[u] : p;
             float x[R::kElems];
@@ -802,7 +815,7 @@ __global__ __launch_bounds__(kThreads) void fused_single_kernel(
         for (int w = 1; w < kW; ++w) M = fmaxf(M, s_max[w]);
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const float p = exp2_fast(s[u] - M);
+            const float p = exp2_fast(below_max(s[u], M));
             l += p;
             const float pv = R::k8bit ? p * t.vs[u] : p;
             float x[R::kElems];
