@@ -817,12 +817,13 @@ def gemv_cpu_baseline(seconds=3.0):
 
 def kernel_key(plan, B, NH, total, append=False, paged=False, ragged=False):
     """(name prefix, grid suffix) of the BF16 split kernel a plan launches, as keyed in the
-    rocprof summaries: `split_kernel<1, MODE, WAVES, TILE, APPEND, PAGED> grid=WORKITEMS`.
+    rocprof summaries: `split_kernel<1, MODE, WAVES, TILE, APPEND, PAGED, NT> grid=WORKITEMS`.
     4 waves in both shapes of this build; TILE (8-row chunks per lane) is 4 in the latency
     shape (B*NH*total below 2^19 rows, `total` the planned attended length) and 8 in the
-    streaming shape and in the device-planned designated kernel (mode 4).  Modes: 0 partials, 1 last-block, 2 cooperative, 3 designated, 4
+    streaming shape.  Modes: 0 partials, 1 last-block, 2 cooperative, 3 designated, 4
     designated planned on the device, 5 partials of ragged lengths on half the grid (two
-    packed segments per workgroup)."""
+    packed segments per workgroup).  NT (non-temporal loads) is false for contiguous
+    designated calls of at most 10 MiB of K and V."""
     st, slots, rows = plan
     tile = 4 if B * NH * total < (1 << 19) else 8
     mode = {2: 0, 4: 0, 5: 1, 3: 2, 6: 3}.get(st)
@@ -831,13 +832,12 @@ def kernel_key(plan, B, NH, total, append=False, paged=False, ragged=False):
     blocks = B * NH * slots
     if mode == 3 and B * NH >= 8:
         blocks = 8 * ((B * NH + 7) // 8) * slots   # designated grid laid out per XCD, padded to 8 heads
-    if mode == 3 and rows == -2 and not paged:
+    if mode == 3 and rows == -1 and not paged:
         mode = 4
     elif mode == 0 and ragged and rows != 0 and B <= 256:
         mode, blocks = 5, (blocks + 1) // 2
-    if mode == 4:
-        tile = 8
-    flags = f"{'true' if append else 'false'}, {'true' if paged else 'false'}"
+    plain = mode in (3, 4) and tile == 4 and not paged and B * NH * total * 256 <= 10 << 20
+    flags = ", ".join("true" if f else "false" for f in (append, paged, not plain))
     return f"split_kernel<1, {mode}, 4, {tile}, {flags}>", f"grid={blocks * 256}"
 
 

@@ -52,8 +52,8 @@ def _key(row) -> str:
     return f"{short_name(row['Kernel_Name'])} grid={grid}"
 
 
-OWN_KERNELS = ("split_kernel", "merge_kernel", "fused_single_kernel", "cache_write", "gemv_kernel",
-               "set_len_kernel")
+OWN_KERNELS = ("split_kernel", "merge_kernel", "fused_single_kernel", "cache_write", "gemv_kernel", "gemm_kernel",
+               "gemm_tall_kernel", "set_len_kernel")
 
 
 def _phases(d: str):
