@@ -11,7 +11,7 @@
 //
 // What bounds it: at the per-layer sizes (0.6 to 4.7 MB of BF16 weights) launch and the first memory
 // round trip (768 x 768, 16 tokens: 3.0 us, of 2.0 for an almost empty launch; 10.5 on the vector
-// units), so K is split over 8 waves until one block of loads per wave covers it, and
+// units), so K is split over 8 waves (up to rows of 1536 bytes one block of loads each), and
 // tiles stay 16 x 16 for the most workgroups.
 //
 // How the operands are read: lane 16 g + r of an MFMA operand holds 16 bytes of row r at K chunk

@@ -92,8 +92,7 @@ __device__ __forceinline__ size_t cache_row(const GemvArgs& a, int b, int part, 
 // dwords of preloaded arguments: W, x, the scales, the bias, M and K, all its first loads
 // need; B and out follow.
 // kPre: several vectors over a row of one block; the next vector's x is requested before this
-// one's products, else each vector waits a round trip to L2 (768 x 3072, us: BF16 2 vectors 4.34,
-// 3.71 with; FP32 5 vectors 8.17, 6.37 with).
+// one's products, else each vector waits a round trip to L2 (where it pays: pre_pays).
 template <int WT, int kC, int kR, bool kOutF32, int kEpi, bool kPre = false>
 __global__ __launch_bounds__(kGemvWaves * kWave) void gemv_kernel(const uint8_t* pk_W, const uint8_t* pk_x,
                                                                   const float* pk_w_scale, const void* pk_bias,
