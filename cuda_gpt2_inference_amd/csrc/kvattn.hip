@@ -164,8 +164,12 @@ __device__ __forceinline__ void decode(const uint4& d, float (&x)[Row<DT>::kElem
 // to an fp32 accumulator) on the packed q pairs that convert_q<DT, true> leaves in q[0..3],
 // then the scale in q[4].  The streaming kernel keeps the fma form: measured, the dot costs
 // its 64-sequence call 2 % (A/B, both the one-chain and the two-chain form).
+// kAlike: every lane of a row gets the same score.  The scale's product may otherwise be fused into
+// the sum over the lanes, each of which then rounds its own: within FP32's error of the score, but
+// not the same number, so only lanes that keep a maximum of their own may take it (fusing it
+// everywhere but there, 12-layer BF16 stack at 1024 positions: 49.6 us, 49.9 without).
 typedef __bf16 Bf16x2 __attribute__((ext_vector_type(2)));
-template <int DT, bool kHw = false>
+template <int DT, bool kHw = false, bool kAlike = false>
 __device__ __forceinline__ float dot_chunk(const float (&q)[Row<DT>::kElems], const uint4& d) {
     if constexpr (kHw && DT == KVATTN_KV_BF16) {
         auto pair = [](uint32_t u) { return __builtin_bit_cast(Bf16x2, u); };
@@ -174,10 +178,10 @@ __device__ __forceinline__ float dot_chunk(const float (&q)[Row<DT>::kElems], co
         s = __builtin_amdgcn_fdot2_f32_bf16(pair(d.y), qp(1), s, false);
         s = __builtin_amdgcn_fdot2_f32_bf16(pair(d.z), qp(2), s, false);
         s = __builtin_amdgcn_fdot2_f32_bf16(pair(d.w), qp(3), s, false);
-        // The lanes of a row add these up: fused into that sum, each lane would round its own product
-        // differently, and they would hold different scores.
-        {
+        if constexpr (kAlike) {
 #pragma clang fp contract(off)
+            return s * q[4];
+        } else {
             return s * q[4];
         }
     } else {
@@ -802,7 +806,7 @@ __global__ __launch_bounds__(kThreads) void fused_single_kernel(
         float mloc = kStartMax;
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            s[u] = row_sum<R::kLanes>(dot_chunk<DT, true>(q, t.k[u]));
+            s[u] = row_sum<R::kLanes>(dot_chunk<DT, true, true>(q, t.k[u]));
             if constexpr (R::k8bit) s[u] *= t.ks[u];
             if (r + u * kRPL + slot_row < total) mloc = fmaxf(mloc, s[u]);
             else s[u] = -INFINITY;
